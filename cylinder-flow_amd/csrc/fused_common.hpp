@@ -261,4 +261,35 @@ __device__ __forceinline__ void pull(const typename S::T *__restrict__ A, const 
     });
 }
 
+// FP64 moments and collision of one node in the reference's term order (3D MPI+KOKKOS+MPIIO/
+// lbm.cpp:390-397, then :257-272): p += f/3.0 per direction, relaxation f - (f - feq)/tau,
+// partial bounce-back with solid fraction sf.
+template <int Q, bool FORCE, bool SFRAC>
+__device__ __forceinline__ void collide_f64(const double *gv, double sf, double tau, double rtau, double *c, double &p,
+                                            double &u, double &v, double &w, double &fx, double &fy, double &fz) {
+    using L = Lat<Q>;
+    p = u = v = w = 0.0;
+    static_for<0, Q>([&](auto I) {
+        constexpr int i = I;
+        p = p + div_cr(gv[i], 3.0, 1.0 / 3.0);
+        if constexpr (L::ex(i) > 0) u = u + gv[i];
+        else if constexpr (L::ex(i) < 0) u = u - gv[i];
+        if constexpr (L::ey(i) > 0) v = v + gv[i];
+        else if constexpr (L::ey(i) < 0) v = v - gv[i];
+        if constexpr (L::ez(i) > 0) w = w + gv[i];
+        else if constexpr (L::ez(i) < 0) w = w - gv[i];
+    });
+    if constexpr (FORCE && SFRAC) {
+        fx += 2.0 * sf * u;
+        fy += 2.0 * sf * v;
+        fz += 2.0 * sf * w;
+    }
+    static_for<0, Q>([&](auto I) {
+        constexpr int i = I;
+        const double feq = feq_ref<Q, i>(p, u, v, w);
+        c[i] = gv[i] - div_cr(gv[i] - feq, tau, rtau);
+        if constexpr (SFRAC) c[i] = (1.0 - sf) * c[i] + sf * gv[L::opp(i)];
+    });
+}
+
 }  // namespace lbm

@@ -92,6 +92,43 @@ hipError_t plain_step(int Q, int prec, int V, const StepBufs &b, bool force, boo
 hipError_t fast_step_f32(int Q, int V, const StepBufs &b, bool force, bool mac, const FusedArgs &a, hipStream_t s);
 hipError_t fast_step_f16(int Q, int V, const StepBufs &b, bool force, bool mac, const FusedArgs &a, hipStream_t s);
 hipError_t fast_step_bf16(int Q, int V, const StepBufs &b, bool force, bool mac, const FusedArgs &a, hipStream_t s);
+// two D3Q27 steps per pass over memory (pair_kernel.hpp): WX x WY columns over runs of cz planes.
+// The words and lists are built once from the mask (pair_plan).
+struct PairPlan {
+    bool on = false;
+    int tiles_x = 0, tiles_y = 0, cz = 0, chunks = 0;
+    uint32_t *bw = nullptr;       // per node (padded layout): bit i set when direction i bounces back
+    uint32_t *tflag = nullptr;    // per column, (nz + 31) / 32 words: bit k set when plane k of the column
+                                  // and its rim holds a non-zero bw
+    // Force partials in the slots of the one-step path of the domain, so that the sums are the same:
+    // one per node next to the mask (nlink of them, node order) ...
+    uint32_t *link = nullptr;     // the nodes ...
+    uint32_t *linklk = nullptr;   // ... their mask links (bit i: direction i pulls from a solid node) ...
+    int *link_slot = nullptr;     // ... and slots (0, 1, ...)
+    int nlink = 0;
+    // ... or one per block of fbx nodes of a row (fgx per row) that holds such a node
+    uint32_t *fblk = nullptr;     // the blocks in slot order (null: per node)
+    int fbx = 0, fgx = 0;
+    int nslots = 0;
+    double *partials = nullptr;   // the slots, then their chunk sums
+};
+struct PairOps {   // a storage format's column, LDS bytes and launchers
+    int wx, wy;
+    size_t lds;
+    hipError_t (*prepare)();
+    hipError_t (*step)(const PairPlan &p, const void *A, void *B, const void *sfrac, const double *uin, double *macros,
+                       bool mac, const FusedArgs &a, hipStream_t s);
+    hipError_t (*force)(const PairPlan &p, const void *A, double *partials, const FusedArgs &a, hipStream_t s);
+};
+PairOps pair_ops(int prec);
+// the plan of a domain; p.on stays false where the two-step kernel does not apply (pair.cpp).
+// flags: on the device, complete on stream s; near_nodes: the nodes next to the mask, in node order;
+// block_slot: the one-step path's slot per block of shape `blk` (empty: its slots are per node)
+hipError_t pair_plan(PairPlan &p, int prec, const Geo &g, const uint8_t *flags, bool same_offsets,
+                     const std::vector<uint32_t> &near_nodes, const std::vector<int> &block_slot, Shape blk, hipStream_t s);
+// fills p.bw, p.tflag and p.linklk (pair_words.hip)
+hipError_t pair_words(const PairPlan &p, const PairOps &ops, const uint8_t *flags, const Geo &g, hipStream_t s);
+void pair_free(PairPlan &p);
 // several D2Q9 FP64 steps per launch (small_kernels.hip): tb_depth() steps at most, T x T tiles
 // (tb_tile), tb_tiles(g, T, K) blocks with tb_lds_bytes(T) of LDS each; tb_prepare() before use
 // bounce-back links of a node for k_tb2d: bit i-1 when direction i pulls from a solid node
@@ -217,6 +254,7 @@ struct lbm_ctx {
     uint32_t *linklk = nullptr;     // words and force slots (for k_link_force)
     int *link_slot = nullptr;
     int nlink = 0;
+    lbm::PairPlan pair;             // D3Q27: two steps per pass
     int V = 1;                      // nodes per lane of the fused kernel
     bool aligned_pull = true;
     bool dense = false;             // FP32/16-bit: per-node pass over every node (see StepBufs)
@@ -242,9 +280,10 @@ struct lbm_ctx {
     // Fields (and, in reference mode, the populations after Update) are written on request, not
     // every step: fields_fresh says they belong to the current state; otherwise replay_ok says the
     // last step's input buffer is intact, so rerunning that step with the moments on rewrites the
-    // same populations and fills them in.
+    // same populations and fills them in (replay_pair: that pass was two steps).
     bool fields_fresh = true;
     bool replay_ok = false;
+    bool replay_pair = false;
     // snapshot staging: device buffer (plain mode) and pinned host buffer, kept for reuse
     double *snap_dev = nullptr, *snap_host = nullptr;
     size_t snap_elems = 0;

@@ -117,6 +117,7 @@ static void free_all(lbm_ctx *c) {
     c->rsurf = nullptr;
     c->nsurf = 0;
     c->rusr = nullptr;
+    pair_free(c->pair);
     if (c->snap_host) (void)hipHostFree(c->snap_host);
     c->snap_host = nullptr;
     c->snap_elems = 0;
@@ -430,6 +431,7 @@ static int init_plain(lbm_ctx *c) {
         return c->solid[(size_t)x + (size_t)g.nx * ((size_t)y + (size_t)g.ny * z)] != 0;
     };
     c->solid_nodes = c->near_nodes = 0;
+    std::vector<uint32_t> near_list;   // D3Q27: the nodes next to the mask
     for (int z = 0; z < g.nz; z++)
         for (int y = 0; y < g.ny; y++)
             for (int x = 0; x < g.nx; x++) {
@@ -443,6 +445,7 @@ static int init_plain(lbm_ctx *c) {
                 for (int i = 1; i < Q && !near; i++) near = solid_at(x - e[3 * i], y - e[3 * i + 1], z - e[3 * i + 2]);
                 flags[node] = near ? FL_NEAR : FL_FLUID;
                 c->near_nodes += near;
+                if (near && Q == 27) near_list.push_back((uint32_t)node);
             }
     const int V = c->V;
     const bool sf = !c->sfrac.empty();
@@ -627,6 +630,15 @@ static int init_plain(lbm_ctx *c) {
     HIP_TRY(c, hipMalloc(&c->block_slot, sizeof(int) * std::max<size_t>(slot.size(), 1)));
     HIP_TRY(c, hipMalloc(&c->partials, sizeof(double) * 3 * (std::max(c->nslots, 1) + force_chunks(c->nslots))));
     HIP_TRY(c, hipMemcpyAsync(c->flags, flags.data(), g.plane, hipMemcpyHostToDevice, c->stream));
+    // D3Q27: two steps per pass over memory where the two-step kernel applies (pair.cpp); its force
+    // slots are those of the one-step path
+    if (Q == 27) {
+        const bool same_offsets = c->prec == LBM_FP64 || c->prec == LBM_FP32 || c->cfg.store_uref == 0.0;
+        const bool per_block = c->prec == LBM_FP64 || c->dense;
+        HIP_TRY(c, pair_plan(c->pair, c->prec, g, c->flags, same_offsets, per_block || sf ? std::vector<uint32_t>() : near_list,
+                             per_block && !sf ? slot : std::vector<int>(), c->prec == LBM_FP64 ? fp64_shape(g, Q) : lane_shape(g, 1),
+                             c->stream));
+    }
     {   // rows whose nodes are all fluid with no solid neighbour (the adjoint's straight-line rows;
         // LBM_ADJ_GENERAL_PATH=1 sends every row through the general path, for tests)
         std::vector<uint8_t> clean((size_t)g.ny * g.nz, std::getenv("LBM_ADJ_GENERAL_PATH") ? 0 : 1);
@@ -844,9 +856,30 @@ static int step_n(lbm_ctx *c, int n, hipEvent_t *evs = nullptr) {
         c->replay_ok = false;
     }
     HIP_TRY(c, tb_force_flush(c->tb_partials, a.g, c->tb_t, c->tb_k, c->hist, rec0, pend, step1, fi, c->stream));
-    for (int k = n - left; k < n; k++) {
+    auto records = [&](long step) { return fi > 0 && step % fi == 0; };
+    while (left > 0) {
+        // two steps in one pass unless the second records the force (its input stays in the LDS), or
+        // the first does and a solid fraction carries force (its moments do too); not under
+        // per-kernel timing
+        if (c->pair.on && !evs && left > 1 && !records(c->step + 2) && !(records(c->step + 1) && c->dsfrac)) {
+            const PairOps ops = pair_ops(c->prec);
+            if (records(c->step + 1)) {
+                HIP_TRY(c, ops.force(c->pair, c->A, c->pair.partials, a, c->stream));
+                HIP_TRY(c, force_reduce(c->pair.partials, c->pair.nslots, c->pair.partials + 3 * (size_t)c->pair.nslots, c->hist,
+                                        c->nrec++, c->step + 1, c->stream));
+            }
+            HIP_TRY(c, ops.step(c->pair, c->A, c->B, c->dsfrac, c->duin, c->macros, false, a, c->stream));
+            c->step += 2;
+            left -= 2;
+            std::swap(c->A, c->B);
+            c->fields_fresh = false;
+            c->replay_ok = c->replay_pair = true;
+            continue;
+        }
+        const int k = n - left;
         c->step++;
-        const bool force = fi > 0 && c->step % fi == 0;
+        left--;
+        const bool force = records(c->step);
         StepBufs b = step_bufs(c, c->A, c->B);
         if (evs) {
             b.ev_bulk[0] = evs[2 * k];
@@ -857,6 +890,7 @@ static int step_n(lbm_ctx *c, int n, hipEvent_t *evs = nullptr) {
         std::swap(c->A, c->B);
         c->fields_fresh = false;
         c->replay_ok = true;
+        c->replay_pair = false;
     }
     return LBM_OK;
 }
@@ -873,7 +907,8 @@ int ensure_fields(lbm_ctx *c) {
         HIP_TRY(c, ref_fused(c->rg, c->rft, c->rf, c->rmac, c->rusr, c->rprof, c->rfpre, c->stream));
     } else {
         const FusedArgs a = ctx_fused_args(c);
-        HIP_TRY(c, plain_step(c->Q, c->prec, c->V, step_bufs(c, c->B, c->A), false, true, a, c->stream));
+        if (c->replay_pair) HIP_TRY(c, pair_ops(c->prec).step(c->pair, c->B, c->A, c->dsfrac, c->duin, c->macros, true, a, c->stream));
+        else HIP_TRY(c, plain_step(c->Q, c->prec, c->V, step_bufs(c, c->B, c->A), false, true, a, c->stream));
     }
     c->fields_fresh = true;
     return LBM_OK;

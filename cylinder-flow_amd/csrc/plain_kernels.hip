@@ -100,30 +100,10 @@ __global__ void __launch_bounds__(512)
     if constexpr (SFRAC) sf = live ? sfrac[node] : (C)0;
     double mp, mu, mv, mw;
     if constexpr (sizeof(C) == 8) {
-        // FP64: the reference's term order -- p += f/3.0 per direction (lbm.cpp:390-397)
-        double p = 0.0, u = 0.0, v = 0.0, w = 0.0;
-        static_for<0, Q>([&](auto I) {
-            constexpr int i = I;
-            p = p + div_cr(gv[i], 3.0, 1.0 / 3.0);
-            if constexpr (L::ex(i) > 0) u = u + gv[i];
-            else if constexpr (L::ex(i) < 0) u = u - gv[i];
-            if constexpr (L::ey(i) > 0) v = v + gv[i];
-            else if constexpr (L::ey(i) < 0) v = v - gv[i];
-            if constexpr (L::ez(i) > 0) w = w + gv[i];
-            else if constexpr (L::ez(i) < 0) w = w - gv[i];
-        });
-        if constexpr (FORCE && SFRAC) {
-            fx += 2.0 * sf * u;
-            fy += 2.0 * sf * v;
-            fz += 2.0 * sf * w;
-        }
-        static_for<0, Q>([&](auto I) {
-            constexpr int i = I;
-            const double feq = feq_ref<Q, i>(p, u, v, w);
-            double c = gv[i] - div_cr(gv[i] - feq, a.tau, a.rtau);
-            if constexpr (SFRAC) c = (1.0 - sf) * c + sf * gv[L::opp(i)];
-            if (live) S::template store<i, L>(B + (size_t)i * g.ds + pnode, c, a.sp);
-        });
+        // FP64: the reference's term order
+        double p, u, v, w, c[Q];
+        collide_f64<Q, FORCE, SFRAC>(gv, sf, a.tau, a.rtau, c, p, u, v, w, fx, fy, fz);
+        if (live) static_for<0, Q>([&](auto I) { S::template store<I, L>(B + (size_t)I * g.ds + pnode, c[I], a.sp); });
         mp = p; mu = u; mv = v; mw = w;
     } else {
         float s = 0.f, u = 0.f, v = 0.f, w = 0.f;
