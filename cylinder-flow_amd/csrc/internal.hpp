@@ -129,22 +129,24 @@ hipError_t pair_plan(PairPlan &p, int prec, const Geo &g, const uint8_t *flags, 
 // fills p.bw, p.tflag and p.linklk (pair_words.hip)
 hipError_t pair_words(const PairPlan &p, const PairOps &ops, const uint8_t *flags, const Geo &g, hipStream_t s);
 void pair_free(PairPlan &p);
-// several D2Q9 FP64 steps per launch (small_kernels.hip): tb_depth() steps at most, T x T tiles
-// (tb_tile), tb_tiles(g, T, K) blocks with tb_lds_bytes(T) of LDS each; tb_prepare() before use
+// several D2Q9 steps per launch (small_kernel.hpp): tb_depth() steps at most, T x T tiles
+// (tb_tile), tb_tiles(g, T, K) blocks with tb_lds_bytes(prec, T) of LDS each
 // bounce-back links of a node for k_tb2d: bit i-1 when direction i pulls from a solid node
 // (after the outlet's clamp), bit 7+i when it pulls across a wall (not for the inlet's unknowns)
 std::vector<uint16_t> tb_links(const Geo &g, const std::vector<uint8_t> &flags);
 int tb_depth();
-size_t tb_lds_bytes(int T);
+size_t tb_lds_bytes(int prec, int T);
 int tb_tiles(const Geo &g, int T, int K, int *tiles_x);
 int tb_tile(const Geo &g, int K, int cus);
-hipError_t tb_prepare();
+// before the first launch: the LDS limit of the kernels for side T (sfrac: null or not) on this device
+hipError_t tb_prepare(int prec, int T, const void *sfrac, const FusedArgs &a);
 // tb_steps: `steps` (<= K) steps in one launch; the partials of its force records go to record
 // slots pend, pend + 1, ... of `partials` (tb_records() slots of ntiles * 3 doubles); *nrec = their
 // count.  tb_force_flush sums npend slots into hist[rec0 ...], the first at step step1.
 int tb_records(int K);
-hipError_t tb_steps(const void *A, void *B, const uint8_t *flags, const uint16_t *lk, const double *uin, double *partials, int pend,
-                    int *nrec, const FusedArgs &a, int T, int K, int steps, long step0, int fi, hipStream_t s);
+hipError_t tb_steps(int prec, const void *A, void *B, const uint8_t *flags, const uint16_t *lk, const void *sfrac,
+                    const double *uin, double *partials, int pend, int *nrec, const FusedArgs &a, int T, int K, int steps,
+                    long step0, int fi, hipStream_t s);
 hipError_t tb_force_flush(const double *partials, const Geo &g, int T, int K, double *hist, int rec0, int npend,
                           long step1, int fi, hipStream_t s);
 // sum of the nslots force partials into hist[rec] (chunks: force_chunks(nslots) * 3 doubles)
@@ -241,7 +243,7 @@ struct lbm_ctx {
     int *block_slot = nullptr;
     double *partials = nullptr;
     int nslots = 0;
-    int tb_k = 0;                   // D2Q9 FP64 small domains: steps per temporally blocked launch (0: off)
+    int tb_k = 0;                   // D2Q9 small domains: steps per temporally blocked launch (0: off)
     int tb_t = 0;                   // and its tile side
     double *tb_partials = nullptr;  // their per-tile force partials (tb_records(tb_k) record slots)
     uint16_t *tb_lk = nullptr;      // and each node's bounce-back links (tb_links)

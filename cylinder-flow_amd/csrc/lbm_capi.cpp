@@ -594,22 +594,31 @@ static int init_plain(lbm_ctx *c) {
             HIP_TRY(c, hipMemcpy(c->link_slot, lslot.data(), sizeof(int) * lslot.size(), hipMemcpyHostToDevice));
         }
     }
-    // D2Q9 FP64 on a small domain, where a step costs about a dependent launch: several steps
-    // per launch (temporal blocking, small_kernels.hip), for walls, inlet, outlet and a mask,
-    // when the population buffer is at most 24 MB (measured against one launch per step: 2.3x
-    // at 3 MB, 1.08x at 17.6 MB, even at 34 MB, slower above); LBM_TEMPORAL_BLOCKING=0 / 1
-    // forbids / allows it regardless of the size.
+    // D2Q9 on a small domain, where a step costs about a dependent launch: several steps per launch
+    // (temporal blocking, small_kernel.hpp), for walls, inlet, outlet, a mask and a solid fraction,
+    // up to 349 525 nodes (padded; 24 MB per FP64 buffer).  us per step with drag every 10 steps, one
+    // launch per step / several: 400x100 FP64 4.64 / 2.00, FP32 4.03 / 1.36, FP16 4.11 / 1.46; 800x200
+    // 7.62 / 5.62, 5.37 / 2.73, 5.01 / 2.96; 1000x250 9.73 / 7.76, 6.39 / 4.68, 5.70 / 5.11; 1400x350
+    // 15.7 / 14.4, 9.2 / 7.8, 8.3 / 8.6.  LBM_TEMPORAL_BLOCKING=0 / 1 forbids / allows it
+    // regardless of the size.
     {
         const char *tbe = std::getenv("LBM_TEMPORAL_BLOCKING");
-        const bool eligible = Q == 9 && c->prec == LBM_FP64 && !g.xper && !g.yper && !sf;
+        // (FP32/16-bit: not under a switch that selects among the one-step kernels, and only where
+        // opposite directions share their storage offset, as a bounced value is taken as stored)
+        bool eligible = Q == 9 && !g.xper && !g.yper;
+        if (c->prec != LBM_FP64) {
+            for (const char *k : {"LBM_FORCE_SLOW_PATH", "LBM_DENSE", "LBM_ALIGNED_PULL", "LBM_NODES_PER_LANE", "LBM_FAST_BLOCKS_PER_CU"})
+                eligible = eligible && std::getenv(k) == nullptr;
+            eligible = eligible && (c->prec == LBM_FP32 || c->cfg.store_uref == 0.0);
+        }
         const bool small = (size_t)8 * Q * g.plane <= ((size_t)24 << 20);
         int dev = 0, lds_max = 0, cus = 0;
         if (eligible && (tbe ? tbe[0] == '1' : small) && hipGetDevice(&dev) == hipSuccess &&
             hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess &&
-            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
-            tb_prepare() == hipSuccess) {
+            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess) {
             const int K = tb_depth(), T = tb_tile(g, K, cus);
-            if ((size_t)lds_max >= tb_lds_bytes(T) + 4096 + 512) {   // + the kernel's static force records
+            if ((size_t)lds_max >= tb_lds_bytes(c->prec, T) + 4096 + 512 &&
+                tb_prepare(c->prec, T, sf ? c : nullptr, ctx_fused_args(c)) == hipSuccess) {   // + the kernel's static force records
                 c->tb_k = K;
                 c->tb_t = T;
                 int tiles_x = 0;
@@ -845,7 +854,7 @@ static int step_n(lbm_ctx *c, int n, hipEvent_t *evs = nullptr) {
             step1 = (c->step + fi) / fi * fi;   // the first force step after the current one
         }
         int nr = 0;
-        HIP_TRY(c, tb_steps(c->A, c->B, c->flags, c->tb_lk, c->duin, c->tb_partials, pend, &nr, a, c->tb_t, c->tb_k, kk, c->step, fi,
+        HIP_TRY(c, tb_steps(c->prec, c->A, c->B, c->flags, c->tb_lk, c->dsfrac, c->duin, c->tb_partials, pend, &nr, a, c->tb_t, c->tb_k, kk, c->step, fi,
                             c->stream));
         pend += nr;
         c->nrec += nr;
