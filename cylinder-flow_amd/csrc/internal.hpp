@@ -142,13 +142,32 @@ int tb_tile(const Geo &g, int K, int cus);
 hipError_t tb_prepare(int prec, int T, const void *sfrac, const FusedArgs &a);
 // tb_steps: `steps` (<= K) steps in one launch; the partials of its force records go to record
 // slots pend, pend + 1, ... of `partials` (tb_records() slots of ntiles * 3 doubles); *nrec = their
-// count.  tb_force_flush sums npend slots into hist[rec0 ...], the first at step step1.
+// count.
 int tb_records(int K);
 hipError_t tb_steps(int prec, const void *A, void *B, const uint8_t *flags, const uint16_t *lk, const void *sfrac,
                     const double *uin, double *partials, int pend, int *nrec, const FusedArgs &a, int T, int K, int steps,
                     long step0, int fi, hipStream_t s);
-hipError_t tb_force_flush(const double *partials, const Geo &g, int T, int K, double *hist, int rec0, int npend,
-                          long step1, int fi, hipStream_t s);
+// sums npend record slots (of `slots`) of nparts triples each into hist[rec0 ...], the first at step step1
+hipError_t tb_force_flush(const double *partials, int nparts, int slots, double *hist, int rec0, int npend, long step1, int fi,
+                          hipStream_t s);
+// several D2Q9 steps per pass over memory on large domains (strip_kernel.hpp): `steps` (2..4) steps
+// from A into B by nwaves waves, strips (66 - 2 steps columns each) x runs of `rows` rows; bit l of rec:
+// step l + 1 records the force, its partials go to record slot pend, pend + 1, ... (nwaves triples each)
+struct StripLaunch {
+    const void *A;
+    void *B;
+    const uint16_t *lk;   // tb_links
+    const void *sfrac;
+    const double *uin;
+    double *partials;
+    int steps, strips, rows, nwaves, pend;
+    uint32_t rec;
+};
+constexpr int STRIP_K = 4;   // steps per pass
+hipError_t strip_launch(int prec, const StripLaunch &l, const FusedArgs &a, hipStream_t s);
+// fills steps, strips, rows and nwaves
+void strip_shape(const Geo &g, int prec, int cus, int steps, StripLaunch &l);
+
 // sum of the nslots force partials into hist[rec] (chunks: force_chunks(nslots) * 3 doubles)
 int force_chunks(int nslots);
 hipError_t force_reduce(const double *partials, int nslots, double *chunks, double *hist, int rec, long step,
@@ -245,7 +264,9 @@ struct lbm_ctx {
     int nslots = 0;
     int tb_k = 0;                   // D2Q9 small domains: steps per temporally blocked launch (0: off)
     int tb_t = 0;                   // and its tile side
-    double *tb_partials = nullptr;  // their per-tile force partials (tb_records(tb_k) record slots)
+    bool strip = false;             // D2Q9 large domains: STRIP_K steps per pass (strip_kernel.hpp)
+    int cus = 0;                    // compute units of the device
+    double *tb_partials = nullptr;  // force partials per tile or wave (tb_records(...) record slots)
     uint16_t *tb_lk = nullptr;      // and each node's bounce-back links (tb_links)
     uint32_t *fix = nullptr;        // FP32/16-bit: nodes recomputed per node after the packed path
     uint32_t *fixlk = nullptr;      // their link words

@@ -113,6 +113,7 @@ static void free_all(lbm_ctx *c) {
     c->tb_partials = nullptr;
     c->tb_lk = nullptr;
     c->tb_k = 0;
+    c->strip = false;
     c->rf = c->rft = c->rmac = c->rprof = c->rfpre = nullptr;
     c->rsurf = nullptr;
     c->nsurf = 0;
@@ -596,38 +597,62 @@ static int init_plain(lbm_ctx *c) {
     }
     // D2Q9 on a small domain, where a step costs about a dependent launch: several steps per launch
     // (temporal blocking, small_kernel.hpp), for walls, inlet, outlet, a mask and a solid fraction,
-    // up to 349 525 nodes (padded; 24 MB per FP64 buffer).  us per step with drag every 10 steps, one
-    // launch per step / several: 400x100 FP64 4.64 / 2.00, FP32 4.03 / 1.36, FP16 4.11 / 1.46; 800x200
-    // 7.62 / 5.62, 5.37 / 2.73, 5.01 / 2.96; 1000x250 9.73 / 7.76, 6.39 / 4.68, 5.70 / 5.11; 1400x350
-    // 15.7 / 14.4, 9.2 / 7.8, 8.3 / 8.6.  LBM_TEMPORAL_BLOCKING=0 / 1 forbids / allows it
+    // up to 420 000 nodes (padded).  On larger ones, and where an axis is periodic, STRIP_K steps per
+    // pass over memory (strip_kernel.hpp), from 360 000 nodes on, in 16-bit storage from 3 million.
+    // us per step with drag every 10 steps, one launch per step / tiles / strips:
+    //               FP64                 FP32                 FP16
+    //   600x150     5.76 / 3.74 / 8.3    4.68 / 1.86 / 5.4    4.47 / 1.95 / 5.8
+    //   1000x250    9.80 / 7.96 / 11.2   6.38 / 4.60 / 6.2    5.64 / 5.06 / 6.6
+    //   1200x300    12.0 / 10.6 / 11.5   7.84 / 5.67 / 6.3    6.82 / 6.41 / 6.7
+    //   1400x350    15.8 / 14.7 / 12.9   9.26 / 7.70 / 7.5    8.28 / 8.65 / 8.5
+    //   2000x500    27.3 / 29.3 / 19.7   15.1 / 15.2 / 10.1   9.99 / 15.9 / 12.0
+    //   2048x2048   100 / 110 / 55.4     50.4 / 56.6 / 24.5   27.0 / 59.8 / 25.1
+    // LBM_TEMPORAL_BLOCKING=0 keeps one step per launch, 1 / 2 take the tiles / the strips
     // regardless of the size.
     {
         const char *tbe = std::getenv("LBM_TEMPORAL_BLOCKING");
         // (FP32/16-bit: not under a switch that selects among the one-step kernels, and only where
         // opposite directions share their storage offset, as a bounced value is taken as stored)
-        bool eligible = Q == 9 && !g.xper && !g.yper;
+        bool eligible = Q == 9;
         if (c->prec != LBM_FP64) {
             for (const char *k : {"LBM_FORCE_SLOW_PATH", "LBM_DENSE", "LBM_ALIGNED_PULL", "LBM_NODES_PER_LANE", "LBM_FAST_BLOCKS_PER_CU"})
                 eligible = eligible && std::getenv(k) == nullptr;
             eligible = eligible && (c->prec == LBM_FP32 || c->cfg.store_uref == 0.0);
         }
-        const bool small = (size_t)8 * Q * g.plane <= ((size_t)24 << 20);
-        int dev = 0, lds_max = 0, cus = 0;
-        if (eligible && (tbe ? tbe[0] == '1' : small) && hipGetDevice(&dev) == hipSuccess &&
-            hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess &&
-            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess) {
-            const int K = tb_depth(), T = tb_tile(g, K, cus);
+        const bool small = g.plane <= 420000, tiles_ok = eligible && !g.xper && !g.yper;
+        const bool large = g.plane >= (c->prec == LBM_FP64 || c->prec == LBM_FP32 ? 360000u : 3000000u);
+        const size_t esz9 = c->prec == LBM_FP64 ? 8 : c->prec == LBM_FP32 ? 4 : 2;
+        int dev = 0, lds_max = 0;
+        if (eligible && (hipGetDevice(&dev) != hipSuccess ||
+                         hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess ||
+                         hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess))
+            eligible = false;
+        int nparts = 0, slots = 0;
+        if (eligible && tiles_ok && (tbe ? tbe[0] == '1' : small)) {
+            const int K = tb_depth(), T = tb_tile(g, K, c->cus);
             if ((size_t)lds_max >= tb_lds_bytes(c->prec, T) + 4096 + 512 &&
-                tb_prepare(c->prec, T, sf ? c : nullptr, ctx_fused_args(c)) == hipSuccess) {   // + the kernel's static force records
+                tb_prepare(c->prec, T, sf ? c : nullptr, ctx_fused_args(c)) == hipSuccess) {
                 c->tb_k = K;
                 c->tb_t = T;
                 int tiles_x = 0;
-                const int nt = tb_tiles(g, T, K, &tiles_x);
-                HIP_TRY(c, hipMalloc(&c->tb_partials, sizeof(double) * 3 * (size_t)nt * tb_records(K)));
-                const std::vector<uint16_t> lk = tb_links(g, flags);
-                HIP_TRY(c, hipMalloc(&c->tb_lk, sizeof(uint16_t) * lk.size()));
-                HIP_TRY(c, hipMemcpy(c->tb_lk, lk.data(), sizeof(uint16_t) * lk.size(), hipMemcpyHostToDevice));
+                nparts = tb_tiles(g, T, K, &tiles_x);
+                slots = tb_records(K);
             }
+        } else if (eligible && (tbe ? tbe[0] == '2' : large) && g.ds == (size_t)g.nxp && esz9 * Q * g.plane < ((size_t)1 << 32)) {
+            // (byte offsets in 32 bits)
+            c->strip = true;
+            for (int k = 2; k <= STRIP_K; k++) {
+                StripLaunch l{};
+                strip_shape(g, c->prec, c->cus, k, l);
+                nparts = std::max(nparts, l.nwaves);
+            }
+            slots = tb_records(STRIP_K);
+        }
+        if (nparts > 0) {
+            HIP_TRY(c, hipMalloc(&c->tb_partials, sizeof(double) * 3 * (size_t)nparts * slots));
+            const std::vector<uint16_t> lk = tb_links(g, flags);
+            HIP_TRY(c, hipMalloc(&c->tb_lk, sizeof(uint16_t) * lk.size()));
+            HIP_TRY(c, hipMemcpy(c->tb_lk, lk.data(), sizeof(uint16_t) * lk.size(), hipMemcpyHostToDevice));
         }
     }
     const size_t esz = c->prec == LBM_FP64 ? 8 : c->prec == LBM_FP32 ? 4 : 2;
@@ -843,19 +868,42 @@ static int step_n(lbm_ctx *c, int n, hipEvent_t *evs = nullptr) {
     int left = n;
     int pend = 0, rec0 = 0;
     long step1 = 0;
-    while (c->tb_k > 0 && !evs && left > 1) {
-        const int kk = std::min(c->tb_k, left - 1);
-        if (pend + kk > tb_records(c->tb_k)) {
-            HIP_TRY(c, tb_force_flush(c->tb_partials, a.g, c->tb_t, c->tb_k, c->hist, rec0, pend, step1, fi, c->stream));
+    auto records = [&](long step) { return fi > 0 && step % fi == 0; };
+    const int depth = c->tb_k > 0 ? c->tb_k : c->strip ? STRIP_K : 0, slots = tb_records(depth);
+    int nparts = 0, tiles_x = 0;   // partials per record of the pending records
+    if (c->tb_k > 0) nparts = tb_tiles(a.g, c->tb_t, c->tb_k, &tiles_x);
+    while (depth > 0 && !evs && left > (c->strip ? 2 : 1)) {
+        const int kk = std::min(depth, left - 1);
+        StripLaunch l{};
+        if (c->strip) strip_shape(a.g, c->prec, c->cus, kk, l);
+        if (pend + kk > slots || (c->strip && pend > 0 && l.nwaves != nparts)) {
+            HIP_TRY(c, tb_force_flush(c->tb_partials, nparts, slots, c->hist, rec0, pend, step1, fi, c->stream));
             pend = 0;
         }
+        if (c->strip) nparts = l.nwaves;
         if (pend == 0 && fi > 0) {
             rec0 = c->nrec;
             step1 = (c->step + fi) / fi * fi;   // the first force step after the current one
         }
         int nr = 0;
-        HIP_TRY(c, tb_steps(c->prec, c->A, c->B, c->flags, c->tb_lk, c->dsfrac, c->duin, c->tb_partials, pend, &nr, a, c->tb_t, c->tb_k, kk, c->step, fi,
-                            c->stream));
+        if (c->strip) {
+            l.A = c->A;
+            l.B = c->B;
+            l.lk = c->tb_lk;
+            l.sfrac = c->dsfrac;
+            l.uin = c->duin;
+            l.partials = c->tb_partials;
+            l.pend = pend;
+            for (int j = 0; j < kk; j++)
+                if (records(c->step + j + 1)) {
+                    l.rec |= 1u << j;
+                    nr++;
+                }
+            HIP_TRY(c, strip_launch(c->prec, l, a, c->stream));
+        } else {
+            HIP_TRY(c, tb_steps(c->prec, c->A, c->B, c->flags, c->tb_lk, c->dsfrac, c->duin, c->tb_partials, pend, &nr, a, c->tb_t,
+                                c->tb_k, kk, c->step, fi, c->stream));
+        }
         pend += nr;
         c->nrec += nr;
         c->step += kk;
@@ -864,8 +912,7 @@ static int step_n(lbm_ctx *c, int n, hipEvent_t *evs = nullptr) {
         c->fields_fresh = false;
         c->replay_ok = false;
     }
-    HIP_TRY(c, tb_force_flush(c->tb_partials, a.g, c->tb_t, c->tb_k, c->hist, rec0, pend, step1, fi, c->stream));
-    auto records = [&](long step) { return fi > 0 && step % fi == 0; };
+    HIP_TRY(c, tb_force_flush(c->tb_partials, nparts, slots, c->hist, rec0, pend, step1, fi, c->stream));
     while (left > 0) {
         // two steps in one pass unless the second records the force (its input stays in the LDS), or
         // the first does and a solid fraction carries force (its moments do too); not under

@@ -104,6 +104,33 @@ __device__ __forceinline__ void buf_store(__amdgpu_buffer_rsrc_t r, uint32_t lan
     }
 }
 
+// bit i of w ? a : b, with the bit spread over a mask (the compiler would compare and select)
+__device__ __forceinline__ uint32_t pair_pick32(uint32_t m, uint32_t a, uint32_t b) {
+    uint32_t r;
+    asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(r) : "v"(m), "v"(a), "v"(b));
+    return r;
+}
+template <class V>
+__device__ __forceinline__ V pair_pick(uint32_t w, int i, V a, V b) {
+    const uint32_t m = (uint32_t)__builtin_amdgcn_sbfe((int)w, i, 1);
+    V r;
+    if constexpr (sizeof(V) == 8) {
+        uint32_t x[2], y[2];
+        __builtin_memcpy(x, &a, 8);
+        __builtin_memcpy(y, &b, 8);
+        x[0] = pair_pick32(m, x[0], y[0]);
+        x[1] = pair_pick32(m, x[1], y[1]);
+        __builtin_memcpy(&r, x, 8);
+    } else {
+        typename UInt<sizeof(V)>::type x, y;
+        __builtin_memcpy(&x, &a, sizeof(V));
+        __builtin_memcpy(&y, &b, sizeof(V));
+        x = (decltype(x))pair_pick32(m, x, y);
+        __builtin_memcpy(&r, &x, sizeof(V));
+    }
+    return r;
+}
+
 // LDS between threads of the block, nothing else: outstanding loads and stores of global memory
 // stay in flight across it
 __device__ __forceinline__ void lds_barrier() {
@@ -185,32 +212,6 @@ struct PairMarch {
     __device__ __forceinline__ uint32_t word(int k, uint32_t node) const {
         const uint32_t on = (tf[k >> 5] >> (k & 31)) & 1u;
         return buf_load<uint32_t>(plane_rsrc(bw + (size_t)planen * k, on * planen * 4u), node * 4u, 0);
-    }
-    // bit i of w ? a : b, with the bit spread over a mask (the compiler would compare and select)
-    __device__ __forceinline__ static uint32_t pick32(uint32_t m, uint32_t a, uint32_t b) {
-        uint32_t r;
-        asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(r) : "v"(m), "v"(a), "v"(b));
-        return r;
-    }
-    template <class V>
-    __device__ __forceinline__ static V pick(uint32_t w, int i, V a, V b) {
-        const uint32_t m = (uint32_t)__builtin_amdgcn_sbfe((int)w, i, 1);
-        V r;
-        if constexpr (sizeof(V) == 8) {
-            uint32_t x[2], y[2];
-            __builtin_memcpy(x, &a, 8);
-            __builtin_memcpy(y, &b, 8);
-            x[0] = pick32(m, x[0], y[0]);
-            x[1] = pick32(m, x[1], y[1]);
-            __builtin_memcpy(&r, x, 8);
-        } else {
-            typename UInt<sizeof(V)>::type x, y;
-            __builtin_memcpy(&x, &a, sizeof(V));
-            __builtin_memcpy(&y, &b, sizeof(V));
-            x = (decltype(x))pick32(m, x, y);
-            __builtin_memcpy(&r, &x, sizeof(V));
-        }
-        return r;
     }
     // whether any lane of the wave holds one of these bits
     __device__ __forceinline__ static bool any(uint32_t bits) { return __builtin_amdgcn_ballot_w64(bits != 0u) != 0ull; }
@@ -319,7 +320,7 @@ struct PairMarch {
                     constexpr int i = I;
                     const uint32_t nom = rr[L::ey(i) + 1] + co[L::ex(i) + 1] + ((L::ez(i) > 0 ? sm : L::ez(i) < 0 ? sp : s0) + i * dsb);
                     const uint32_t own = here + (s0 + L::opp(i) * dsb);
-                    R[i] = buf_load<T>(rs, pick<uint32_t>(w, i, own, nom), 0);
+                    R[i] = buf_load<T>(rs, pair_pick<uint32_t>(w, i, own, nom), 0);
                 });
             } else {
                 static_for<0, Q>([&](auto I) {
@@ -350,7 +351,7 @@ struct PairMarch {
                 constexpr int i = I;
                 if constexpr (L::ez(i) < 0) {
                     const T o = ownv[zrank(i) * WX * WY];
-                    r[i] = pick<T>(w2, i, o, r[i]);
+                    r[i] = pair_pick<T>(w2, i, o, r[i]);
                 }
             });
         C g[Q], c[Q], s, u, v, w;
@@ -383,8 +384,8 @@ struct PairMarch {
             static_for<1, Q>([&](auto I) {
                 constexpr int i = I;
                 const T o = in[L::opp(i) * NP + i0];
-                if constexpr (L::ez(i) == 0) midJ[zrank(i)] = pick<T>(w2, i, o, midJ[zrank(i)]);
-                else if constexpr (L::ez(i) > 0) upJ[zrank(i)] = pick<T>(w2, i, o, upJ[zrank(i)]);
+                if constexpr (L::ez(i) == 0) midJ[zrank(i)] = pair_pick<T>(w2, i, o, midJ[zrank(i)]);
+                else if constexpr (L::ez(i) > 0) upJ[zrank(i)] = pair_pick<T>(w2, i, o, upJ[zrank(i)]);
                 else if (act2) ownv[zrank(i) * WX * WY] = o;
             });
     }

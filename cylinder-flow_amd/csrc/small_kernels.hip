@@ -2,6 +2,7 @@
 // launches and the sum of its force records.
 #include "small_kernel.hpp"
 
+#include <algorithm>
 #include <cstdlib>
 
 namespace lbm {
@@ -81,24 +82,28 @@ int tb_tile(const Geo &g, int K, int cus) {
 std::vector<uint16_t> tb_links(const Geo &g, const std::vector<uint8_t> &flags) {
     using L = Lat<9>;
     std::vector<uint16_t> lk(flags.size(), 0);
-    for (int y = 0; y < g.ny; y++)
+    for (int y = 0; y < g.ny; y++) {
+        const bool wallrow = !g.yper && (y == 0 || y == g.ny - 1);
         for (int x = 0; x < g.nx; x++) {
             const size_t node = (size_t)x + (size_t)g.nxp * y;
-            if (flags[node] == FL_SOLID) continue;
+            if (flags[node] == FL_SOLID || (!wallrow && flags[node] != FL_NEAR)) continue;
             uint16_t b = 0;
             for (int i = 1; i < 9; i++) {
                 const int ex = L::ex(i), ey = L::ey(i);
-                if (ex > 0 && x == 0) continue;                            // Zou-He unknown
-                const int sy = y - ey;
+                if (ex > 0 && x == 0 && !g.xper) continue;                 // Zou-He unknown
+                int sx = x - ex, sy = y - ey;
+                if (g.yper) sy = (sy + g.ny) % g.ny;
                 if (sy < 0 || sy >= g.ny) {                                // wall
                     b |= (uint16_t)(1u << (7 + i));
                     continue;
                 }
-                const int sx = (ex < 0 && x == g.nx - 1) ? x : x - ex;     // outlet clamp
+                if (g.xper) sx = (sx + g.nx) % g.nx;
+                else if (sx == g.nx) sx = x;                               // outlet clamp
                 if (flags[(size_t)sx + (size_t)g.nxp * sy] == FL_SOLID) b |= (uint16_t)(1u << (i - 1));
             }
             lk[node] = b;
         }
+    }
     return lk;
 }
 
@@ -142,14 +147,38 @@ hipError_t tb_steps(int prec, const void *A, void *B, const uint8_t *flags, cons
                                     nforce > 0, false}, a, s);
 }
 
-hipError_t tb_force_flush(const double *partials, const Geo &g, int T, int K, double *hist, int rec0, int npend,
-                          long step1, int fi, hipStream_t s) {
+hipError_t tb_force_flush(const double *partials, int nparts, int slots, double *hist, int rec0, int npend, long step1, int fi,
+                          hipStream_t s) {
     if (npend <= 0) return hipSuccess;
-    if (npend > tb_records(K) || fi <= 0) return hipErrorInvalidValue;
-    int tiles_x = 0;
-    const int ntiles = tb_tiles(g, T, K, &tiles_x);
-    hipLaunchKernelGGL(k_tb_force, dim3(npend), dim3(256), 0, s, partials, ntiles, hist, rec0, step1, fi);
+    if (npend > slots || fi <= 0) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_tb_force, dim3(npend), dim3(256), 0, s, partials, nparts, hist, rec0, step1, fi);
     return hipGetLastError();
+}
+
+hipError_t strip_launch_f64(const StripLaunch &l, const FusedArgs &a, hipStream_t s);
+hipError_t strip_launch_f32(const StripLaunch &l, const FusedArgs &a, hipStream_t s);
+hipError_t strip_launch_f16(const StripLaunch &l, const FusedArgs &a, hipStream_t s);
+hipError_t strip_launch_bf16(const StripLaunch &l, const FusedArgs &a, hipStream_t s);
+
+hipError_t strip_launch(int prec, const StripLaunch &l, const FusedArgs &a, hipStream_t s) {
+    switch (prec) {
+    case LBM_FP64: return strip_launch_f64(l, a, s);
+    case LBM_FP32: return strip_launch_f32(l, a, s);
+    case LBM_FP16S: return strip_launch_f16(l, a, s);
+    case LBM_BF16S: return strip_launch_bf16(l, a, s);
+    default: return hipErrorInvalidValue;
+    }
+}
+
+void strip_shape(const Geo &g, int prec, int cus, int steps, StripLaunch &l) {
+    l.steps = steps;
+    l.strips = (g.nx + 65 - 2 * steps) / (66 - 2 * steps);
+    // a run per resident wave (2 per SIMD with FP64's registers, 4 otherwise), but no run shorter than
+    // 4 rows: it would recompute more rows than it stores
+    const int res = prec == LBM_FP64 ? 2 : 4, per_run = l.strips + (g.xper ? 0 : 1);
+    const int runs = std::max(1, cus * 4 * res / per_run);
+    l.rows = std::max((g.ny + runs - 1) / runs, 4);
+    l.nwaves = per_run * ((g.ny + l.rows - 1) / l.rows);
 }
 
 }  // namespace lbm

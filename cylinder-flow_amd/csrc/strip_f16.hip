@@ -1,0 +1,8 @@
+// strip_f16.hip -- the large-domain D2Q9 kernel of strip_kernel.hpp for SF16 storage
+#include "strip_kernel.hpp"
+
+namespace lbm {
+
+hipError_t strip_launch_f16(const StripLaunch &l, const FusedArgs &a, hipStream_t s) { return strip_launch_s<SF16>(l, a, s); }
+
+}  // namespace lbm
