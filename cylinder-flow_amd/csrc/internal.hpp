@@ -184,6 +184,9 @@ hipError_t count_nonfinite(int prec, const void *base, size_t sy, size_t sz, int
 // moment plane k (p, u, v, w) at the physical nodes; 0 at solid nodes
 hipError_t macros_extract(const double *macros, const uint8_t *flags, double *out, int k, const Geo &g, hipStream_t s);
 
+// the moment planes of mask (bit k: p, u, v, w) one after another, physical nodes, 0 at solid nodes
+hipError_t plain_fields(const double *macros, const uint8_t *flags, double *out, unsigned mask, const Geo &g, hipStream_t s);
+
 // ---- reference mode (FP64, ghost-padded SoA) ----
 struct RefGeo {
     int Q, D, g;                 // ghost width 3 (3D) / 2 (2D)
@@ -213,6 +216,8 @@ hipError_t ref_stream(const RefGeo &r, const double *f, double *ft, hipStream_t 
 hipError_t ref_update(const RefGeo &r, double *f, double *mac, const uint8_t *usr, const double *prof, double *fpre,
                       hipStream_t s);
 int ref_mem_blocks(const RefGeo &r);
+// the interior (ghost layers stripped) of the moment planes of mask, one after another
+hipError_t ref_fields(const RefGeo &r, const double *mac, double *out, unsigned mask, hipStream_t s);
 
 // ---- adjoint (plain mode) ----
 struct AdjArgs {
@@ -307,6 +312,11 @@ struct lbm_ctx {
     bool fields_fresh = true;
     bool replay_ok = false;
     bool replay_pair = false;
+    // results on their way to the caller (output.cpp): device buffer and pinned memory, kept for reuse,
+    // and the force records already on the host
+    double *out_dev = nullptr, *out_pin = nullptr;
+    size_t out_elems = 0, out_pinned = 0;
+    std::vector<double> hist_copy;
     // snapshot staging: device buffer (plain mode) and pinned host buffer, kept for reuse
     double *snap_dev = nullptr, *snap_host = nullptr;
     size_t snap_elems = 0;
@@ -320,5 +330,11 @@ struct lbm_ctx {
 
 // materialise the fields of the last step (see lbm_capi.cpp); LBM_OK or an LBM_ERR_* code
 int ensure_fields(lbm_ctx *c);
+// device results into the caller's arrays (output.cpp)
+hipError_t output_fields(lbm_ctx *c, double *const *outs);
+hipError_t output_stage(lbm_ctx *c, double **dev);
+hipError_t output_staged(lbm_ctx *c, double *dst);
+hipError_t output_forces(lbm_ctx *c);
+void output_free(lbm_ctx *c);
 // the address of lbm_get_fields_noalloc's staging array on the current device (noalloc.hip)
 int noalloc_setup(double **out, std::string &err);

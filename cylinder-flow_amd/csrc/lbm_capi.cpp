@@ -119,6 +119,7 @@ static void free_all(lbm_ctx *c) {
     c->nsurf = 0;
     c->rusr = nullptr;
     pair_free(c->pair);
+    output_free(c);
     if (c->snap_host) (void)hipHostFree(c->snap_host);
     c->snap_host = nullptr;
     c->snap_elems = 0;
@@ -1101,8 +1102,8 @@ extern "C" int lbm_sync(lbm_ctx *c) {
     HIP_TRY(c, hipStreamSynchronize(c->stream));
     if (c->nrec > c->nrec_checked) {
         const int k = c->nrec - c->nrec_checked;
-        std::vector<double> h(4 * (size_t)k);
-        HIP_TRY(c, hipMemcpy(h.data(), c->hist + 4 * (size_t)c->nrec_checked, h.size() * sizeof(double), hipMemcpyDeviceToHost));
+        HIP_TRY(c, output_forces(c));
+        const double *const h = c->hist_copy.data() + 4 * (size_t)c->nrec_checked;
         const int first = c->nrec_checked;
         c->nrec_checked = c->nrec;
         for (int r = 0; r < k; r++)
@@ -1165,30 +1166,7 @@ extern "C" int lbm_get_fields(lbm_ctx *c, double *p, double *u, double *v, doubl
         const int rc = ensure_fields(c);
         if (rc != LBM_OK) return rc;
     }
-    if (ref_mode(c->cfg.bc_mode)) {
-        std::vector<double> pad(c->rg.plane);
-        for (int k = 0; k < 4; k++) {
-            if (!outs[k]) continue;
-            HIP_TRY(c, hipMemcpyAsync(pad.data(), c->rmac + (size_t)k * c->rg.plane, sizeof(double) * c->rg.plane,
-                                      hipMemcpyDeviceToHost, c->stream));
-            HIP_TRY(c, hipStreamSynchronize(c->stream));
-            ref_strip(c, pad, outs[k]);
-        }
-        return LBM_OK;
-    }
-    double *tmp = nullptr;
-    HIP_TRY(c, hipMalloc(&tmp, sizeof(double) * c->N));
-    for (int k = 0; k < 4; k++) {
-        if (!outs[k]) continue;
-        hipError_t e = macros_extract(c->macros, c->flags, tmp, k, c->geo, c->stream);
-        if (e == hipSuccess) e = hipMemcpyAsync(outs[k], tmp, sizeof(double) * c->N, hipMemcpyDeviceToHost, c->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-        if (e != hipSuccess) {
-            (void)hipFree(tmp);
-            return set_err(c, LBM_ERR_HIP, std::string("lbm_get_fields: ") + hipGetErrorString(e));
-        }
-    }
-    (void)hipFree(tmp);
+    HIP_TRY(c, output_fields(c, outs));
     return LBM_OK;
 }
 
@@ -1216,17 +1194,11 @@ extern "C" int lbm_get_populations(lbm_ctx *c, double *f) {
     }
     const FusedArgs a = ctx_fused_args(c);
     double *tmp = nullptr;
-    HIP_TRY(c, hipMalloc(&tmp, sizeof(double) * c->N));
+    HIP_TRY(c, output_stage(c, &tmp));
     for (int i = 0; i < c->Q; i++) {
-        hipError_t e = plain_decode(c->Q, c->prec, c->A, tmp, c->flags, i, a, c->stream);
-        if (e == hipSuccess) e = hipMemcpyAsync(f + (size_t)i * c->N, tmp, sizeof(double) * c->N, hipMemcpyDeviceToHost, c->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-        if (e != hipSuccess) {
-            (void)hipFree(tmp);
-            return set_err(c, LBM_ERR_HIP, std::string("lbm_get_populations: ") + hipGetErrorString(e));
-        }
+        HIP_TRY(c, plain_decode(c->Q, c->prec, c->A, tmp, c->flags, i, a, c->stream));
+        HIP_TRY(c, output_staged(c, f + (size_t)i * c->N));
     }
-    (void)hipFree(tmp);
     return LBM_OK;
 }
 
@@ -1257,10 +1229,10 @@ extern "C" int lbm_set_populations(lbm_ctx *c, const double *f) {
 
 extern "C" int lbm_get_forces(lbm_ctx *c, double *out, int max, int *count) {
     if (!c) return LBM_ERR_INVALID;
-    HIP_TRY(c, hipStreamSynchronize(c->stream));
+    HIP_TRY(c, output_forces(c));
     if (count) *count = c->nrec;
     const int n = std::min(max, c->nrec);
-    if (out && n > 0) HIP_TRY(c, hipMemcpy(out, c->hist, sizeof(double) * 4 * (size_t)n, hipMemcpyDeviceToHost));
+    if (out && n > 0) std::memcpy(out, c->hist_copy.data(), sizeof(double) * 4 * (size_t)n);
     return LBM_OK;
 }
 

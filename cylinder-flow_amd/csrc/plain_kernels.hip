@@ -251,6 +251,23 @@ __global__ void __launch_bounds__(512) k_macros_extract(const double *__restrict
     out[(size_t)x + (size_t)g.nx * ((size_t)y + (size_t)g.ny * z)] = flags[node] == FL_SOLID ? 0.0 : mac[node];
 }
 
+// the planes of mask (bits 0..3) in one pass: plane k's values at out + (its rank in mask) * nodes
+__global__ void __launch_bounds__(512) k_plain_fields(const double *__restrict__ mac, const uint8_t *__restrict__ flags,
+                                                      double *__restrict__ out, unsigned mask, Geo g) {
+    const int x = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y, z = blockIdx.z;
+    if (x >= g.nx) return;
+    const size_t row = (size_t)y + (size_t)g.ny * z, node = (size_t)x + (size_t)g.nxp * row;
+    const size_t n = (size_t)g.nx * g.ny * g.nz;
+    const bool solid = flags[node] == FL_SOLID;
+    double *o = out + (size_t)x + (size_t)g.nx * row;
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+        if ((mask >> k) & 1u) {
+            *o = solid ? 0.0 : mac[k * g.plane + node];
+            o += n;
+        }
+}
+
 // Health check of a population buffer (lbm_sync): counts the non-finite values of one direction
 // over a box of nodes, element base + x + sy*y + sz*z (x < nx; y, z the grid), skipping the nodes
 // flagged solid when flags is set (flags at x + fpitch*(y + ny*z)).  A non-finite population
@@ -434,6 +451,12 @@ hipError_t count_nonfinite(int prec, const void *base, size_t sy, size_t sz, int
                            bad);
         return hipGetLastError();
     });
+}
+
+hipError_t plain_fields(const double *macros, const uint8_t *flags, double *out, unsigned mask, const Geo &g, hipStream_t s) {
+    const Shape sh = node_shape(g);
+    hipLaunchKernelGGL(k_plain_fields, grid_of(g, sh), dim3(sh.bx), 0, s, macros, flags, out, mask, g);
+    return hipGetLastError();
 }
 
 hipError_t macros_extract(const double *macros, const uint8_t *flags, double *out, int k, const Geo &g, hipStream_t s) {

@@ -572,6 +572,26 @@ hipError_t ref_fused(const RefGeo &r, const double *f, double *ft, double *mac, 
     return launch_rows<FusedK>(r, s, f, ft, mac, usr, prof, fpre);
 }
 
+__global__ void __launch_bounds__(256) k_ref_fields(const double *__restrict__ mac, RefGeo r, double *__restrict__ out, unsigned mask) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y, k = blockIdx.z;
+    if (i >= r.glx) return;
+    const int gz = r.D == 3 ? r.g : 0;
+    const size_t n = (size_t)(i + r.g) + (size_t)r.px * ((size_t)(j + r.g) + (size_t)r.ly * (k + gz));
+    double *o = out + (size_t)i + (size_t)r.glx * ((size_t)j + (size_t)r.gly * k);
+#pragma unroll
+    for (int m = 0; m < 4; m++)
+        if ((mask >> m) & 1u) {
+            *o = mac[m * r.plane + n];
+            o += (size_t)r.glx * r.gly * r.glz;
+        }
+}
+
+hipError_t ref_fields(const RefGeo &r, const double *mac, double *out, unsigned mask, hipStream_t s) {
+    hipLaunchKernelGGL(k_ref_fields, dim3((unsigned)((r.glx + 255) / 256), (unsigned)r.gly, (unsigned)(r.D == 3 ? r.glz : 1)), dim3(256),
+                       0, s, mac, r, out, mask);
+    return hipGetLastError();
+}
+
 hipError_t ref_stream(const RefGeo &r, const double *f, double *ft, hipStream_t s) {
     return launch_rows<StreamK>(r, s, f, ft);
 }
