@@ -216,6 +216,28 @@ hipError_t ref_stream(const RefGeo &r, const double *f, double *ft, hipStream_t 
 hipError_t ref_update(const RefGeo &r, double *f, double *mac, const uint8_t *usr, const double *prof, double *fpre,
                       hipStream_t s);
 int ref_mem_blocks(const RefGeo &r);
+// One 2D step in one launch: every pulled value straight from where the fills and usrbc would have copied
+// it from (ref_resolve), so neither buffer's ghosts are touched.
+struct RefLink {       // a momentum-exchange link: f_i at the fluid node + f_opp at the solid one
+    int a, b, b0;      // elements of f: the first, the second after usrbc, the second's origin before the fills
+    int dir;
+};
+struct RefOne {
+    bool on = false;
+    int *special = nullptr;     // per node: row of `rows`, -1 where every source is the plain neighbour
+    int *rows = nullptr;        // 9 source elements of each special node
+    RefLink *links = nullptr;   // in node order, directions in order
+    int nlinks = 0;
+};
+// false: some source is a ghost slot that no fill of the same step writes (the values of an earlier
+// step then stay in the ghosts, which only the separate fills keep)
+bool ref_resolve(const RefGeo &r, const std::vector<uint8_t> &usr, std::vector<int> &special, std::vector<int> &rows,
+                 std::vector<RefLink> &links);
+// hist non-null: the force record of the step (from the same input) goes to hist[4 * rec ...]
+hipError_t ref_one(const RefGeo &r, const RefOne &o, const double *f, double *ft, double *mac, const uint8_t *usr,
+                   const double *prof, double *fpre, double *hist, int rec, long step, hipStream_t s);
+// the same sum after the separate fills and usrbc
+hipError_t ref_one_force(const RefGeo &r, const RefOne &o, const double *f, double *hist, int rec, long step, hipStream_t s);
 // the interior (ghost layers stripped) of the moment planes of mask, one after another
 hipError_t ref_fields(const RefGeo &r, const double *mac, double *out, unsigned mask, hipStream_t s);
 
@@ -300,6 +322,7 @@ struct lbm_ctx {
     lbm::RefGeo rg{};
     double *rf = nullptr, *rft = nullptr, *rmac = nullptr, *rprof = nullptr, *rfpre = nullptr;
     uint8_t *rusr = nullptr;
+    lbm::RefOne rone;               // 2D: one launch per step
     uint32_t *rsurf = nullptr;      // interior solid nodes with a fluid neighbour (usrbc's work list)
     int nsurf = 0;
 

@@ -93,7 +93,7 @@ extern "C" const char *lbm_last_error(const lbm_ctx *ctx) { return ctx ? ctx->er
 static void free_all(lbm_ctx *c) {
     void *ptrs[] = {c->A, c->B, c->flags, c->dsfrac, c->duin, c->macros, c->block_slot, c->partials, c->hist, c->fix,
                     c->fixlk, c->rowwin, c->wlk, c->link, c->linklk, c->link_slot, c->rowclean, c->rf, c->rft, c->rmac, c->rprof, c->rusr, c->rfpre, c->rsurf,
-                    c->snap_dev, c->dbad, c->tb_partials, c->tb_lk};
+                    c->snap_dev, c->dbad, c->tb_partials, c->tb_lk, c->rone.special, c->rone.rows, c->rone.links};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     c->A = c->B = nullptr;
@@ -118,6 +118,7 @@ static void free_all(lbm_ctx *c) {
     c->rsurf = nullptr;
     c->nsurf = 0;
     c->rusr = nullptr;
+    c->rone = RefOne{};
     pair_free(c->pair);
     output_free(c);
     if (c->snap_host) (void)hipHostFree(c->snap_host);
@@ -775,6 +776,23 @@ static int init_ref(lbm_ctx *c) {
         if (!surf.empty())
             HIP_TRY(c, hipMemcpy(c->rsurf, surf.data(), sizeof(uint32_t) * surf.size(), hipMemcpyHostToDevice));
     }
+    // 2D: a whole step in one launch where the fills and usrbc can be resolved (one block sums the drag, so
+    // up to 16 384 links)
+    if (c->D == 2) {
+        std::vector<int> special, rows;
+        std::vector<RefLink> links;
+        if (ref_resolve(r, usr, special, rows, links) && links.size() <= 16384) {
+            HIP_TRY(c, hipMalloc(&c->rone.special, sizeof(int) * special.size()));
+            HIP_TRY(c, hipMalloc(&c->rone.rows, sizeof(int) * std::max<size_t>(rows.size(), 1)));
+            HIP_TRY(c, hipMalloc(&c->rone.links, sizeof(RefLink) * std::max<size_t>(links.size(), 1)));
+            HIP_TRY(c, hipMemcpy(c->rone.special, special.data(), sizeof(int) * special.size(), hipMemcpyHostToDevice));
+            HIP_TRY(c, hipMemcpy(c->rone.rows, rows.data(), sizeof(int) * rows.size(), hipMemcpyHostToDevice));
+            if (!links.empty())
+                HIP_TRY(c, hipMemcpy(c->rone.links, links.data(), sizeof(RefLink) * links.size(), hipMemcpyHostToDevice));
+            c->rone.nlinks = (int)links.size();
+            c->rone.on = true;
+        }
+    }
     const int nblk = ref_mem_blocks(r);
     HIP_TRY(c, hipMalloc(&c->partials, sizeof(double) * 3 * nblk));
     c->nslots = nblk;
@@ -832,6 +850,10 @@ StepBufs step_bufs(const lbm_ctx *c, const void *A, void *B) {
 // (launch-bound, the drag every step by default) one pass does both; in 3D usrbc runs over its
 // list and the exchange separately.
 static hipError_t ref_boundary_pass(lbm_ctx *c, bool force) {
+    if (force && c->rone.on) {
+        const hipError_t e = ref_usrbc(c->rg, c->rf, c->rusr, c->rsurf, c->nsurf, c->stream);
+        return e != hipSuccess ? e : ref_one_force(c->rg, c->rone, c->rf, c->hist, c->nrec++, c->step, c->stream);
+    }
     if (force && c->D == 2)
         return ref_mem(c->rg, c->rf, c->rusr, c->partials, c->nslots, c->hist, c->nrec++, c->step, true, c->stream);
     hipError_t e = ref_usrbc(c->rg, c->rf, c->rusr, c->rsurf, c->nsurf, c->stream);
@@ -852,6 +874,15 @@ static int step_n(lbm_ctx *c, int n, hipEvent_t *evs = nullptr) {
         for (int k = 0; k < n; k++) {
             c->step++;
             const bool force = fi > 0 && c->step % fi == 0;
+            if (c->rone.on) {
+                HIP_TRY(c, ref_one(c->rg, c->rone, c->rf, c->rft, nullptr, c->rusr, c->rprof, nullptr, force ? c->hist : nullptr,
+                                   c->nrec, c->step, c->stream));
+                c->nrec += force;
+                std::swap(c->rf, c->rft);
+                c->fields_fresh = false;
+                c->replay_ok = true;
+                continue;
+            }
             HIP_TRY(c, ref_fills(c->rg, c->rf, c->rft, c->stream));
             HIP_TRY(c, ref_boundary_pass(c, force));
             HIP_TRY(c, ref_fused(c->rg, c->rf, c->rft, nullptr, c->rusr, c->rprof, nullptr, c->stream));
@@ -961,7 +992,9 @@ int ensure_fields(lbm_ctx *c) {
     if (c->fields_fresh) return LBM_OK;
     if (!c->replay_ok) return set_err(c, LBM_ERR_STATE, "fields of the current state are not available");
     if (ref_mode(c->cfg.bc_mode)) {
-        HIP_TRY(c, ref_fused(c->rg, c->rft, c->rf, c->rmac, c->rusr, c->rprof, c->rfpre, c->stream));
+        if (c->rone.on)
+            HIP_TRY(c, ref_one(c->rg, c->rone, c->rft, c->rf, c->rmac, c->rusr, c->rprof, c->rfpre, nullptr, 0, 0, c->stream));
+        else HIP_TRY(c, ref_fused(c->rg, c->rft, c->rf, c->rmac, c->rusr, c->rprof, c->rfpre, c->stream));
     } else {
         const FusedArgs a = ctx_fused_args(c);
         if (c->replay_pair) HIP_TRY(c, pair_ops(c->prec).step(c->pair, c->B, c->A, c->dsfrac, c->duin, c->macros, true, a, c->stream));

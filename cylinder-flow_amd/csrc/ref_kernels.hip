@@ -16,6 +16,9 @@
 // Update_n inside the pull kernel (3D MPI+KOKKOS+MPIIO/main.cpp:29-37).  The fills write
 // every ghost slot into both buffers, so ghost values persist across the swaps exactly as in
 // the reference's single f array -- including the slots no fill ever refreshes.
+#include <algorithm>
+#include <unordered_map>
+
 #include "internal.hpp"
 #include "lattice.hpp"
 
@@ -431,6 +434,87 @@ __global__ void __launch_bounds__(256) k_ref_update(RefGeo r, double *f, double 
     ref_update_collide<Q, NT>(r, i, j, k, n, pe, fv, mac, usr, prof, fpre, f);
 }
 
+// Momentum exchange over the list of links (MPI Kokkos/lbm.cpp:364-392), one block, in a fixed order:
+// thread t sums links t, t + NT, ..., then the block's sum.  RESOLVED: before the fills and usrbc, from the
+// elements they copy.
+template <int NT, bool RESOLVED>
+__device__ __forceinline__ void ref_link_sum(const RefLink *__restrict__ links, int n, const double *__restrict__ f,
+                                             double *__restrict__ hist, int rec, long step) {
+    using L = Lat<9>;
+    double fx = 0.0, fy = 0.0;
+    for (int k = (int)threadIdx.x; k < n; k += NT) {
+        const RefLink l = links[k];
+        const double m = f[l.a] + f[RESOLVED ? l.b0 : l.b];
+        static_for<1, 9>([&](auto I) {
+            if (l.dir == (int)I) {
+                fx += m * (double)L::ex(I);
+                fy += m * (double)L::ey(I);
+            }
+        });
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        fx += __shfl_xor(fx, off);
+        fy += __shfl_xor(fy, off);
+    }
+    __shared__ double red[2 * (NT / 64)];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    if (lane == 0) {
+        red[2 * wv] = fx;
+        red[2 * wv + 1] = fy;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int q = 1; q < NT / 64; q++) {
+            red[0] += red[2 * q];
+            red[1] += red[2 * q + 1];
+        }
+        hist[4 * (size_t)rec] = (double)step;
+        hist[4 * (size_t)rec + 1] = red[0];
+        hist[4 * (size_t)rec + 2] = red[1];
+        hist[4 * (size_t)rec + 3] = 0.0;
+    }
+}
+
+__global__ void __launch_bounds__(128) k_ref_one_force(const RefLink *__restrict__ links, int n, const double *__restrict__ f,
+                                                       double *__restrict__ hist, int rec, long step) {
+    ref_link_sum<128, false>(links, n, f, hist, rec, step);
+}
+
+// A whole 2D step of the reference (fills, usrbc, momentum exchange, stream, Update, next Collision) in one
+// launch, where the sequence takes four or five: these steps are bound by their launches (512x128 with the
+// drag every step: 21.7 us in five launches).  The fills and usrbc only copy; a node one of them reaches
+// reads its sources from a table of their origins, every other node its neighbours.  On force steps
+// the first row of blocks (FORCE, its block 0) sums the exchange from the same input.
+template <bool NT, bool FORCE>
+__global__ void __launch_bounds__(128)
+    k_ref_one(RefGeo r, const int *__restrict__ special, const int *__restrict__ rows, const RefLink *__restrict__ links, int nlinks,
+              const double *__restrict__ f, double *__restrict__ ft, double *__restrict__ mac, const uint8_t *__restrict__ usr,
+              const double *__restrict__ prof, double *__restrict__ fpre, double *__restrict__ hist, int rec, long step) {
+    using L = Lat<9>;
+    constexpr int Q = 9;
+    if (FORCE && blockIdx.y == 0) {
+        if (blockIdx.x == 0) ref_link_sum<128, true>(links, nlinks, f, hist, rec, step);
+        return;
+    }
+    const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x) + r.g, j = (int)blockIdx.y - (FORCE ? 1 : 0) + r.g;
+    if (i >= r.lx - r.g) return;
+    const size_t n = (size_t)i + (size_t)r.px * (size_t)j, pe = RIDX(r, 0, i, j, 0);
+    const int sp = special[n];
+    double fv[Q];
+    if (sp < 0) {
+        static_for<0, Q>([&](auto I) {
+            constexpr int ii = I;
+            fv[ii] = f[RIDX(r, ii, i - L::ex(ii), j - L::ey(ii), 0)];
+        });
+    } else {
+        int at[Q];
+        static_for<0, Q>([&](auto I) { at[I] = rows[Q * (size_t)sp + I]; });
+        static_for<0, Q>([&](auto I) { fv[I] = f[at[I]]; });
+    }
+    ref_update_collide<Q, NT>(r, i, j, 0, n, pe, fv, mac, usr, prof, fpre, ft);
+}
+
 __global__ void __launch_bounds__(256) k_ref_reduce(const double *__restrict__ partials, int n, double *__restrict__ hist,
                                                     int rec, long step) {
     double a = 0.0, b = 0.0, c = 0.0;
@@ -570,6 +654,112 @@ template <int Q, bool NT> struct UpdateK {
 hipError_t ref_fused(const RefGeo &r, const double *f, double *ft, double *mac, const uint8_t *usr,
                      const double *prof, double *fpre, hipStream_t s) {
     return launch_rows<FusedK>(r, s, f, ft, mac, usr, prof, fpre);
+}
+
+bool ref_resolve(const RefGeo &r, const std::vector<uint8_t> &usr, std::vector<int> &special, std::vector<int> &rows,
+                 std::vector<RefLink> &links) {
+    using L = Lat<9>;
+    if (r.D != 2 || r.plane * 9 > (size_t)INT32_MAX) return false;
+    const int lx = r.lx, ly = r.ly, g = r.g;
+    const long plane = (long)r.plane;
+    int e[9][2], opp[9];
+    static_for<0, 9>([&](auto I) {
+        e[I][0] = L::ex(I);
+        e[I][1] = L::ey(I);
+        opp[I] = L::opp(I);
+    });
+    auto at = [&](int ii, int i, int j) { return ii * plane + i + (long)r.px * j; };   // RIDX in 2D, flat as there
+    // the element a copied element's value comes from, after the fills in their order and after usrbc, and
+    // the nodes that pull from a node with a copied element (the fills touch the edges, usrbc the body)
+    std::unordered_map<long, int> from;
+    from.reserve(8 * (size_t)(lx + ly));
+    std::vector<uint8_t> reached(r.plane, 0);
+    std::vector<std::pair<long, int>> copies;
+    auto origin = [&](long k) {
+        const auto it = from.find(k);
+        return it == from.end() ? (int)k : it->second;
+    };
+    auto copy = [&](long dst, long src) { copies.emplace_back(dst, origin(src)); };
+    auto apply = [&]() {   // the copies of one fill read what was there before it
+        for (const auto &c : copies) {
+            from[c.first] = c.second;
+            const int n = (int)(c.first % plane), i = n % r.px, j = n / r.px;
+            for (int b = std::max(j - 1, 0); b <= std::min(j + 1, ly - 1); b++)
+                for (int a = std::max(i - 1, 0); a <= std::min(i + 1, lx - 1); a++) reached[(size_t)a + (size_t)r.px * b] = 1;
+        }
+        copies.clear();
+    };
+    for (int j = 1; j < ly - 1; j++) {   // fill2<0>, fill2<1>
+        for (int ii : {1, 5, 8}) copy(at(ii, 1, j), at(ii, 2, j));
+        for (int ii : {3, 6, 7}) copy(at(ii, lx - 2, j), at(ii, lx - 3, j + e[ii][1]));
+    }
+    apply();
+    for (int i = 1; i < lx - 1; i++) {   // fill2<2>, fill2<3>
+        if (r.variant == 1 && (i < 2 || i >= lx - 2)) continue;
+        for (int ii : {2, 5, 6}) copy(at(ii, i, 1), at(opp[ii], i + 2 * e[ii][0], 3));
+        for (int ii : {4, 7, 8}) copy(at(ii, i, ly - 2), at(opp[ii], i + 2 * e[ii][0], ly - 4));
+    }
+    apply();
+    for (int j = g; j < ly - g; j++)     // usrbc
+        for (int i = g; i < lx - g; i++) {
+            if (usr[(size_t)i + (size_t)r.px * j] != 0) continue;
+            for (int ii = 0; ii < 9; ii++)
+                if (usr[(size_t)(i + e[ii][0]) + (size_t)r.px * (j + e[ii][1])] == 1)
+                    copy(at(ii, i, j), at(opp[ii], i + 2 * e[ii][0], j + 2 * e[ii][1]));
+        }
+    apply();
+    auto interior = [&](int k) {
+        const int n = (int)(k % plane), i = n % r.px, j = n / r.px;
+        return i >= g && i < lx - g && j >= g && j < ly - g;
+    };
+    special.assign(r.plane, -1);
+    rows.clear();
+    links.clear();
+    for (int j = g; j < ly - g; j++)
+        for (int i = g; i < lx - g; i++) {
+            const size_t n = (size_t)i + (size_t)r.px * j;
+            // nothing copied nearby: plain neighbours, all interior unless the node lies on the edge
+            const bool edge = i == g || i == lx - g - 1 || j == g || j == ly - g - 1;
+            if (!reached[n] && !edge) continue;
+            int src[9];
+            bool plain = true;
+            for (int ii = 0; ii < 9; ii++) {
+                const long k = at(ii, i - e[ii][0], j - e[ii][1]);
+                src[ii] = origin(k);
+                plain = plain && src[ii] == (int)k;
+                if (!interior(src[ii])) return false;
+            }
+            if (!plain) {
+                special[n] = (int)(rows.size() / 9);
+                rows.insert(rows.end(), src, src + 9);
+            }
+            if (usr[n] != 1) continue;
+            for (int ii = 1; ii < 9; ii++)
+                if (usr[(size_t)(i + e[ii][0]) + (size_t)r.px * (j + e[ii][1])] == 0) {
+                    const long b = at(opp[ii], i + e[ii][0], j + e[ii][1]);
+                    const int b0 = origin(b);
+                    if (!interior(b0)) return false;
+                    links.push_back({(int)at(ii, i, j), (int)b, b0, ii});
+                }
+        }
+    return true;
+}
+
+hipError_t ref_one(const RefGeo &r, const RefOne &o, const double *f, double *ft, double *mac, const uint8_t *usr,
+                   const double *prof, double *fpre, double *hist, int rec, long step, hipStream_t s) {
+    const dim3 grid((unsigned)((r.glx + 127) / 128), (unsigned)(r.gly + (hist ? 1 : 0)));
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, grid, dim3(128), 0, s, r, o.special, o.rows, o.links, o.nlinks, f, ft, mac, usr, prof, fpre, hist, rec, step);
+    };
+    if (nt_stores(r)) hist ? go(k_ref_one<true, true>) : go(k_ref_one<true, false>);
+    else hist ? go(k_ref_one<false, true>) : go(k_ref_one<false, false>);
+    return hipGetLastError();
+}
+
+hipError_t ref_one_force(const RefGeo &r, const RefOne &o, const double *f, double *hist, int rec, long step, hipStream_t s) {
+    (void)r;
+    hipLaunchKernelGGL(k_ref_one_force, dim3(1), dim3(128), 0, s, o.links, o.nlinks, f, hist, rec, step);
+    return hipGetLastError();
 }
 
 __global__ void __launch_bounds__(256) k_ref_fields(const double *__restrict__ mac, RefGeo r, double *__restrict__ out, unsigned mask) {
