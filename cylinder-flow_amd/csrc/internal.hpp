@@ -50,6 +50,39 @@ struct Shape {
 };
 Shape node_shape(const Geo &g);
 
+// ---- initialisation of the node arrays (setup_kernels.hip) ----
+struct SetupBody {
+    int kind;   // lbm_config::body
+    double cx, cy, cz, r2;
+};
+struct SetupFix {   // the rule of the FP32/16-bit fix list (init_plain); V nodes per lane
+    int V;
+    bool all, same_offsets;
+};
+// a node of the periodic x edges, or one whose lane reaches into the padding
+__host__ __device__ inline bool fix_edge(const Geo &g, int V, int x) {
+    return (g.xper && (x == 0 || x == g.nx - 1)) || (x == g.nx - 1 && g.nx % V != 0);
+}
+// a node of the inlet's or outlet's lane
+__host__ __device__ inline bool fix_end_lane(const Geo &g, int V, int x) {
+    const int x0 = x / V * V;
+    return x0 == 0 || x0 + V >= g.nx;
+}
+// flags (padded layout) from the mask bytes (nx*ny*nz; null: from the body formula); sfrac: the caller's
+// solid fraction on the device (nx*ny*nz) or null; counts: solid nodes, near nodes,
+// nodes of the fix list
+hipError_t setup_flags(int Q, uint8_t *flags, const uint8_t *mask, const double *sfrac, const SetupBody &b, const SetupFix &fix,
+                       const Geo &g, unsigned *counts, hipStream_t s);
+// per block of shape blk: 1 when it holds a node whose links or solid fraction carry force
+hipError_t setup_forced(const uint8_t *flags, const double *sfrac, uint8_t *out, Shape blk, const Geo &g, hipStream_t s);
+// per row: 1 when all its nodes are FL_FLUID
+hipError_t setup_clean(const uint8_t *flags, uint8_t *clean, const Geo &g, hipStream_t s);
+// the solid fraction in the padded layout and the precision of the collision, 0 in the padding
+hipError_t setup_sfrac(int prec, const double *in, void *out, const Geo &g, hipStream_t s);
+// bounce-back links of the nodes for k_tb2d and k_strip: bit i-1 when direction i pulls from a solid node
+// (after the outlet's clamp), bit 7+i when it pulls across a wall (not for the inlet's unknowns)
+hipError_t setup_links9(const uint8_t *flags, uint16_t *lk, const Geo &g, hipStream_t s);
+
 hipError_t plain_init(int Q, int prec, void *A, void *B, double *macros, const uint8_t *flags, const double *uin,
                       const double *xi, double perturb, uint64_t seed, const FusedArgs &a, hipStream_t s);
 // launch shape of the fused kernels: V nodes per lane, at most 256 lanes per block
@@ -131,9 +164,6 @@ hipError_t pair_words(const PairPlan &p, const PairOps &ops, const uint8_t *flag
 void pair_free(PairPlan &p);
 // several D2Q9 steps per launch (small_kernel.hpp): tb_depth() steps at most, T x T tiles
 // (tb_tile), tb_tiles(g, T, K) blocks with tb_lds_bytes(prec, T) of LDS each
-// bounce-back links of a node for k_tb2d: bit i-1 when direction i pulls from a solid node
-// (after the outlet's clamp), bit 7+i when it pulls across a wall (not for the inlet's unknowns)
-std::vector<uint16_t> tb_links(const Geo &g, const std::vector<uint8_t> &flags);
 int tb_depth();
 size_t tb_lds_bytes(int prec, int T);
 int tb_tiles(const Geo &g, int T, int K, int *tiles_x);
@@ -156,7 +186,7 @@ hipError_t tb_force_flush(const double *partials, int nparts, int slots, double 
 struct StripLaunch {
     const void *A;
     void *B;
-    const uint16_t *lk;   // tb_links
+    const uint16_t *lk;   // setup_links9
     const void *sfrac;
     const double *uin;
     double *partials;
@@ -294,7 +324,7 @@ struct lbm_ctx {
     bool strip = false;             // D2Q9 large domains: STRIP_K steps per pass (strip_kernel.hpp)
     int cus = 0;                    // compute units of the device
     double *tb_partials = nullptr;  // force partials per tile or wave (tb_records(...) record slots)
-    uint16_t *tb_lk = nullptr;      // and each node's bounce-back links (tb_links)
+    uint16_t *tb_lk = nullptr;      // and each node's bounce-back links (setup_links9)
     uint32_t *fix = nullptr;        // FP32/16-bit: nodes recomputed per node after the packed path
     uint32_t *fixlk = nullptr;      // their link words
     int nfix = 0;

@@ -361,17 +361,6 @@ static void inlet_profile(const lbm_ctx *c, std::vector<double> &uin) {
         }
 }
 
-static bool body_inside(const lbm_config &cfg, int D, int x, int y, int z) {
-    if (cfg.body != LBM_BODY_SPHERE && cfg.body != LBM_BODY_ZCYL) return false;
-    const double dx = (double)x - cfg.cx, dy = (double)y - cfg.cy;
-    double r = dx * dx + dy * dy;
-    if (D == 3 && cfg.body == LBM_BODY_SPHERE) {
-        const double dz = (double)z - cfg.cz;
-        r = r + dz * dz;
-    }
-    return r <= cfg.r2;
-}
-
 static int grow_hist(lbm_ctx *c, int need) {
     if (need <= c->hist_cap) return LBM_OK;
     int cap = std::max(need, std::max(1024, 2 * c->hist_cap));
@@ -408,73 +397,111 @@ FusedArgs ctx_fused_args(const lbm_ctx *c) {
     return a;
 }
 
+struct DevTmp {   // device memory of a scope
+    void *p = nullptr;
+    DevTmp() = default;
+    DevTmp(const DevTmp &) = delete;
+    ~DevTmp() {
+        if (p) (void)hipFree(p);
+    }
+    hipError_t alloc(size_t n) { return hipMalloc(&p, n); }
+};
+
 static int init_plain(lbm_ctx *c) {
     const Geo &g = c->geo;
-    const int Q = c->Q, D = c->D;
-    // solid mask: the body formula (the reference's "usr", 3D MPI+KOKKOS+MPIIO/lbm.cpp:238) or a user mask
-    if (c->cfg.body == LBM_BODY_MASK) {
-        if (c->solid.size() != c->N) return set_err(c, LBM_ERR_STATE, "body = LBM_BODY_MASK needs lbm_set_mask first");
-    } else {
-        c->solid.assign(c->N, 0);
-        for (int z = 0; z < g.nz; z++)
-            for (int y = 0; y < g.ny; y++)
-                for (int x = 0; x < g.nx; x++)
-                    c->solid[(size_t)x + (size_t)g.nx * ((size_t)y + (size_t)g.ny * z)] = body_inside(c->cfg, D, x, y, z);
-    }
+    const int Q = c->Q;
+    if (c->cfg.body == LBM_BODY_MASK && c->solid.size() != c->N)
+        return set_err(c, LBM_ERR_STATE, "body = LBM_BODY_MASK needs lbm_set_mask first");
     if (!c->uin_set) inlet_profile(c, c->uin);
-    // node flags (padded layout); padding columns are marked solid
     std::vector<int> e(3 * Q), opp(Q);
     lbm_lattice_table(Q, e.data(), nullptr, opp.data());
-    std::vector<uint8_t> flags(g.plane, FL_SOLID);
+    const int V = c->V;
+    const bool sf = !c->sfrac.empty();
+    const char *force_slow = std::getenv("LBM_FORCE_SLOW_PATH");
+    const bool all_slow = c->prec != LBM_FP64 && force_slow && force_slow[0] == '1';
+    const bool same_offsets = c->prec == LBM_FP64 || c->prec == LBM_FP32 || c->cfg.store_uref == 0.0;
+    // node flags, solid fraction and the counts on the device (setup_kernels.hip): from the body formula
+    // (the reference's "usr", 3D MPI+KOKKOS+MPIIO/lbm.cpp:238) or the user mask
+    HIP_TRY(c, hipMalloc(&c->flags, g.plane));
+    unsigned counts[3] = {0, 0, 0};      // solid, near nodes, nodes of the fix list
+    std::vector<uint8_t> forced_blk;     // per block of shape s1: holds a forced node
+    const Shape s1 = c->prec == LBM_FP64 ? fp64_shape(g, Q) : lane_shape(g, 1);
+    bool per_block = c->prec == LBM_FP64;
+    {
+        DevTmp mask, frac, cnt, blk;
+        if (c->cfg.body == LBM_BODY_MASK) {
+            HIP_TRY(c, mask.alloc(c->N));
+            HIP_TRY(c, hipMemcpyAsync(mask.p, c->solid.data(), c->N, hipMemcpyHostToDevice, c->stream));
+        }
+        if (sf) {
+            HIP_TRY(c, frac.alloc(sizeof(double) * c->N));
+            HIP_TRY(c, hipMemcpyAsync(frac.p, c->sfrac.data(), sizeof(double) * c->N, hipMemcpyHostToDevice, c->stream));
+            HIP_TRY(c, hipMalloc(&c->dsfrac, (c->prec == LBM_FP64 ? sizeof(double) : sizeof(float)) * g.plane));
+            HIP_TRY(c, setup_sfrac(c->prec, (const double *)frac.p, c->dsfrac, g, c->stream));
+        }
+        HIP_TRY(c, cnt.alloc(sizeof(counts)));
+        const SetupBody body{c->cfg.body, c->cfg.cx, c->cfg.cy, c->cfg.cz, c->cfg.r2};
+        const SetupFix fx{V, all_slow, same_offsets};
+        HIP_TRY(c, setup_flags(Q, c->flags, (const uint8_t *)mask.p, (const double *)frac.p, body, fx, g, (unsigned *)cnt.p, c->stream));
+        HIP_TRY(c, hipMemcpyAsync(counts, cnt.p, sizeof(counts), hipMemcpyDeviceToHost, c->stream));
+        HIP_TRY(c, hipStreamSynchronize(c->stream));
+        if (c->prec != LBM_FP64) {
+            // Dense mode: one per-node pass over every node instead of the copies, the packed pass
+            // and the fix-up of the list, chosen
+            //  * when the fix list holds more than a quarter of the fluid nodes (a solid fraction
+            //    over a noisy field: half of them on the 192x96x96 adjoint workload, where the
+            //    list path took 67 + 100 us per step and the dense pass 67 us), or
+            //  * when a population buffer is at most 16 MB: such steps are launch-bound, and one
+            //    launch fewer per step counts (D2Q9 512x128 with the drag every step: 6.7 / 6.4 us
+            //    per step in FP32 / FP16 against 8.7 / 8.8; on D3Q27 512x128x128 the dense pass
+            //    is as fast in FP32 but 1.5 times slower in FP16, so large domains keep the list).
+            // LBM_DENSE=1 / 0 forces the choice.
+            const size_t pop_bytes = (size_t)(c->prec == LBM_FP32 ? 4 : 2) * Q * g.plane;
+            const bool small = pop_bytes <= ((size_t)16 << 20);
+            const char *dense_env = std::getenv("LBM_DENSE");
+            c->dense = dense_env ? dense_env[0] == '1' : (!all_slow && ((size_t)counts[2] * 4 > c->N - counts[0] || small));
+            per_block = c->dense;
+        }
+        if (per_block) {
+            forced_blk.resize((size_t)s1.gx * g.ny * g.nz);
+            HIP_TRY(c, blk.alloc(forced_blk.size()));
+            HIP_TRY(c, setup_forced(c->flags, (const double *)frac.p, (uint8_t *)blk.p, s1, g, c->stream));
+            HIP_TRY(c, hipMemcpyAsync(forced_blk.data(), blk.p, forced_blk.size(), hipMemcpyDeviceToHost, c->stream));
+            HIP_TRY(c, hipStreamSynchronize(c->stream));
+        }
+    }
+    c->solid_nodes = (int)counts[0];
+    c->near_nodes = (int)counts[1];
+    // rows whose nodes are all fluid with no solid neighbour (the adjoint's straight-line rows;
+    // LBM_ADJ_GENERAL_PATH=1 sends every row through the general path, for tests)
+    std::vector<uint8_t> clean((size_t)g.ny * g.nz);
+    HIP_TRY(c, hipMalloc(&c->rowclean, clean.size()));
+    HIP_TRY(c, setup_clean(c->flags, c->rowclean, g, c->stream));
+    HIP_TRY(c, hipMemcpyAsync(clean.data(), c->rowclean, clean.size(), hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(c, hipStreamSynchronize(c->stream));
+    // the lists below are per node; a dense or FP64 step needs none
+    std::vector<uint8_t> flags;
+    std::vector<uint32_t> near_list;   // D3Q27: the nodes next to the mask
+    if (!per_block) {
+        flags.resize(g.plane);
+        HIP_TRY(c, hipMemcpyAsync(flags.data(), c->flags, g.plane, hipMemcpyDeviceToHost, c->stream));
+        HIP_TRY(c, hipStreamSynchronize(c->stream));
+    }
     auto solid_at = [&](int x, int y, int z) -> bool {
         if (g.xper) x = (x + g.nx) % g.nx;
         if (g.yper) y = (y + g.ny) % g.ny;
         if (g.zper) z = (z + g.nz) % g.nz;
         if (x < 0 || x >= g.nx || y < 0 || y >= g.ny || z < 0 || z >= g.nz) return false;
-        return c->solid[(size_t)x + (size_t)g.nx * ((size_t)y + (size_t)g.ny * z)] != 0;
-    };
-    c->solid_nodes = c->near_nodes = 0;
-    std::vector<uint32_t> near_list;   // D3Q27: the nodes next to the mask
-    for (int z = 0; z < g.nz; z++)
-        for (int y = 0; y < g.ny; y++)
-            for (int x = 0; x < g.nx; x++) {
-                const size_t node = (size_t)x + (size_t)g.nxp * ((size_t)y + (size_t)g.ny * z);
-                if (solid_at(x, y, z)) {
-                    flags[node] = FL_SOLID;
-                    c->solid_nodes++;
-                    continue;
-                }
-                bool near = false;
-                for (int i = 1; i < Q && !near; i++) near = solid_at(x - e[3 * i], y - e[3 * i + 1], z - e[3 * i + 2]);
-                flags[node] = near ? FL_NEAR : FL_FLUID;
-                c->near_nodes += near;
-                if (near && Q == 27) near_list.push_back((uint32_t)node);
-            }
-    const int V = c->V;
-    const bool sf = !c->sfrac.empty();
-    auto forced = [&](int x, int y, int z) {   // a node whose links or solid fraction carry force
-        if (x >= g.nx) return false;
-        const size_t node = (size_t)x + (size_t)g.nxp * ((size_t)y + (size_t)g.ny * z);
-        return flags[node] == FL_NEAR ||
-               (sf && flags[node] != FL_SOLID && c->sfrac[(size_t)x + (size_t)g.nx * ((size_t)y + (size_t)g.ny * z)] > 0.0);
+        return flags[(size_t)x + (size_t)g.nxp * ((size_t)y + (size_t)g.ny * z)] == FL_SOLID;
     };
     // per-node kernels over every node (FP64 k_fused, dense mode k_dense_v; one node per lane):
     // a force partial slot per block holding a forced node
     std::vector<int> slot;
     c->nslots = 0;
-    auto block_slots = [&]() {
-        const Shape s1 = c->prec == LBM_FP64 ? fp64_shape(g, Q) : lane_shape(g, 1);
-        slot.assign((size_t)s1.gx * g.ny * g.nz, -1);
-        c->nslots = 0;
-        for (int z = 0; z < g.nz; z++)
-            for (int y = 0; y < g.ny; y++)
-                for (int bxi = 0; bxi < s1.gx; bxi++) {
-                    bool any = false;
-                    for (int x = bxi * s1.bx; x < std::min(g.nx, (bxi + 1) * s1.bx) && !any; x++) any = forced(x, y, z);
-                    if (any) slot[(size_t)bxi + (size_t)s1.gx * ((size_t)y + (size_t)g.ny * z)] = c->nslots++;
-                }
-    };
-    if (c->prec == LBM_FP64) block_slots();
+    if (per_block) {
+        slot.resize(forced_blk.size());
+        for (size_t b = 0; b < slot.size(); b++) slot[b] = forced_blk[b] ? c->nslots++ : -1;
+    }
     // FP32/16-bit: per fluid node (row-major padded indices), either
     //  * the link list: mask neighbours whose half-way bounce-back the packed kernel applies
     //    in its pull, from per-row windows of link words and force slots (below), or
@@ -487,26 +514,21 @@ static int init_plain(lbm_ctx *c) {
     // LBM_FORCE_SLOW_PATH=1 puts every fluid node on the fix list.  Force partial slots go to
     // the forced nodes in node order across both lists, so the force sum does not depend on
     // which list a node is on.
-    if (c->prec != LBM_FP64) {
-        const char *force_slow = std::getenv("LBM_FORCE_SLOW_PATH");
-        const bool all_slow = force_slow && force_slow[0] == '1';
-        const bool same_offsets = c->prec == LBM_FP32 || c->cfg.store_uref == 0.0;
+    if (!per_block) {
         std::vector<uint32_t> fix, fixlk, link, linklk;
         std::vector<int> lslot;
-        size_t fluid = 0;
         for (int z = 0; z < g.nz; z++)
-            for (int y = 0; y < g.ny; y++)
+            for (int y = 0; y < g.ny; y++) {
+                if (!sf && !all_slow && !g.xper && g.nx % V == 0 && clean[(size_t)y + (size_t)g.ny * z]) continue;   // nothing listed
                 for (int x = 0; x < g.nx; x++) {
                     const size_t node = (size_t)x + (size_t)g.nxp * ((size_t)y + (size_t)g.ny * z);
                     if (flags[node] == FL_SOLID) continue;
-                    fluid++;
-                    const bool f = forced(x, y, z), near = flags[node] == FL_NEAR;
+                    const bool near = flags[node] == FL_NEAR;
                     const bool sfr = sf && c->sfrac[(size_t)x + (size_t)g.nx * ((size_t)y + (size_t)g.ny * z)] > 0.0;
-                    const bool edge = (g.xper && (x == 0 || x == g.nx - 1)) || (x == g.nx - 1 && g.nx % V != 0);
-                    const int x0 = x / V * V;   // first node of the packed kernel's lane
-                    const bool end_lane = x0 == 0 || x0 + V >= g.nx;
-                    const bool to_fix = all_slow || sfr || edge || (near && (end_lane || !same_offsets));
+                    const bool f = near || sfr;   // a node whose links or solid fraction carry force
+                    const bool to_fix = all_slow || sfr || fix_edge(g, V, x) || (near && (fix_end_lane(g, V, x) || !same_offsets));
                     if (!to_fix && !near) continue;
+                    if (near && Q == 27) near_list.push_back((uint32_t)node);
                     // link word: the per-node pull's classification (Zou-He unknowns and wall
                     // links first, outlet clamp, periodic wrap), bit i when the source is solid
                     uint32_t bits = 0;
@@ -532,28 +554,7 @@ static int init_plain(lbm_ctx *c) {
                         lslot.push_back(k);
                     }
                 }
-        // Dense mode: one per-node pass over every node instead of the copies, the packed pass
-        // and the fix-up of the list, chosen
-        //  * when the fix list holds more than a quarter of the fluid nodes (a solid fraction
-        //    over a noisy field: half of them on the 192x96x96 adjoint workload, where the
-        //    list path took 67 + 100 us per step and the dense pass 67 us), or
-        //  * when a population buffer is at most 16 MB: such steps are launch-bound, and one
-        //    launch fewer per step counts (D2Q9 512x128 with the drag every step: 6.7 / 6.4 us
-        //    per step in FP32 / FP16 against 8.7 / 8.8; on D3Q27 512x128x128 the dense pass
-        //    is as fast in FP32 but 1.5 times slower in FP16, so large domains keep the list).
-        // LBM_DENSE=1 / 0 forces the choice.
-        const size_t pop_bytes = (size_t)(c->prec == LBM_FP32 ? 4 : 2) * Q * g.plane;
-        const bool small = pop_bytes <= ((size_t)16 << 20);
-        const char *dense_env = std::getenv("LBM_DENSE");
-        c->dense = dense_env ? dense_env[0] == '1' : (!all_slow && (fix.size() * 4 > fluid || small));
-        if (c->dense) {
-            fix.clear();
-            fixlk.clear();
-            link.clear();
-            linklk.clear();
-            lslot.clear();
-            block_slots();
-        }
+            }
         if (fix.size() > (size_t)INT32_MAX || link.size() > (size_t)INT32_MAX)
             return set_err(c, LBM_ERR_INVALID, "too many boundary nodes");
         c->nfix = (int)fix.size();
@@ -652,36 +653,28 @@ static int init_plain(lbm_ctx *c) {
         }
         if (nparts > 0) {
             HIP_TRY(c, hipMalloc(&c->tb_partials, sizeof(double) * 3 * (size_t)nparts * slots));
-            const std::vector<uint16_t> lk = tb_links(g, flags);
-            HIP_TRY(c, hipMalloc(&c->tb_lk, sizeof(uint16_t) * lk.size()));
-            HIP_TRY(c, hipMemcpy(c->tb_lk, lk.data(), sizeof(uint16_t) * lk.size(), hipMemcpyHostToDevice));
+            HIP_TRY(c, hipMalloc(&c->tb_lk, sizeof(uint16_t) * g.plane));
+            HIP_TRY(c, setup_links9(c->flags, c->tb_lk, g, c->stream));
         }
     }
     const size_t esz = c->prec == LBM_FP64 ? 8 : c->prec == LBM_FP32 ? 4 : 2;
     HIP_TRY(c, hipMalloc(&c->A, esz * Q * g.plane));
     HIP_TRY(c, hipMalloc(&c->B, esz * Q * g.plane));
-    HIP_TRY(c, hipMalloc(&c->flags, g.plane));
     HIP_TRY(c, hipMalloc(&c->duin, sizeof(double) * c->uin.size()));
     HIP_TRY(c, hipMalloc(&c->macros, sizeof(double) * 4 * g.plane));
     HIP_TRY(c, hipMalloc(&c->block_slot, sizeof(int) * std::max<size_t>(slot.size(), 1)));
     HIP_TRY(c, hipMalloc(&c->partials, sizeof(double) * 3 * (std::max(c->nslots, 1) + force_chunks(c->nslots))));
-    HIP_TRY(c, hipMemcpyAsync(c->flags, flags.data(), g.plane, hipMemcpyHostToDevice, c->stream));
     // D3Q27: two steps per pass over memory where the two-step kernel applies (pair.cpp); its force
     // slots are those of the one-step path
     if (Q == 27) {
-        const bool same_offsets = c->prec == LBM_FP64 || c->prec == LBM_FP32 || c->cfg.store_uref == 0.0;
-        const bool per_block = c->prec == LBM_FP64 || c->dense;
-        HIP_TRY(c, pair_plan(c->pair, c->prec, g, c->flags, same_offsets, per_block || sf ? std::vector<uint32_t>() : near_list,
-                             per_block && !sf ? slot : std::vector<int>(), c->prec == LBM_FP64 ? fp64_shape(g, Q) : lane_shape(g, 1),
-                             c->stream));
+        HIP_TRY(c, pair_plan(c->pair, c->prec, g, c->flags, same_offsets, sf ? std::vector<uint32_t>() : near_list,
+                             per_block && !sf ? slot : std::vector<int>(), s1, c->stream));
     }
-    {   // rows whose nodes are all fluid with no solid neighbour (the adjoint's straight-line rows;
-        // LBM_ADJ_GENERAL_PATH=1 sends every row through the general path, for tests)
-        std::vector<uint8_t> clean((size_t)g.ny * g.nz, std::getenv("LBM_ADJ_GENERAL_PATH") ? 0 : 1);
-        for (size_t r = 0; r < clean.size(); r++)
-            for (int x = 0; x < g.nx && clean[r]; x++) clean[r] = flags[(size_t)x + (size_t)g.nxp * r] == FL_FLUID;
-        HIP_TRY(c, hipMalloc(&c->rowclean, clean.size()));
-        HIP_TRY(c, hipMemcpy(c->rowclean, clean.data(), clean.size(), hipMemcpyHostToDevice));
+    {
+        if (std::getenv("LBM_ADJ_GENERAL_PATH")) {
+            std::fill(clean.begin(), clean.end(), (uint8_t)0);
+            HIP_TRY(c, hipMemcpy(c->rowclean, clean.data(), clean.size(), hipMemcpyHostToDevice));
+        }
         c->adj_all_fast = true;
         for (int z = 0; z < g.nz; z++)
             for (int y = 0; y < g.ny; y++) {
@@ -692,20 +685,6 @@ static int init_plain(lbm_ctx *c) {
     HIP_TRY(c, hipMemcpyAsync(c->duin, c->uin.data(), sizeof(double) * c->uin.size(), hipMemcpyHostToDevice, c->stream));
     if (!slot.empty())
         HIP_TRY(c, hipMemcpy(c->block_slot, slot.data(), sizeof(int) * slot.size(), hipMemcpyHostToDevice));
-    if (sf) {
-        const size_t ssz = c->prec == LBM_FP64 ? 8 : 4;
-        std::vector<char> buf(ssz * g.plane, 0);
-        for (int z = 0; z < g.nz; z++)
-            for (int y = 0; y < g.ny; y++)
-                for (int x = 0; x < g.nx; x++) {
-                    const size_t node = (size_t)x + (size_t)g.nxp * ((size_t)y + (size_t)g.ny * z);
-                    const double v = c->sfrac[(size_t)x + (size_t)g.nx * ((size_t)y + (size_t)g.ny * z)];
-                    if (ssz == 8) ((double *)buf.data())[node] = v;
-                    else ((float *)buf.data())[node] = (float)v;
-                }
-        HIP_TRY(c, hipMalloc(&c->dsfrac, buf.size()));
-        HIP_TRY(c, hipMemcpyAsync(c->dsfrac, buf.data(), buf.size(), hipMemcpyHostToDevice, c->stream));
-    }
     double *dxi = nullptr;
     if (!c->xi.empty()) {
         HIP_TRY(c, hipMalloc(&dxi, sizeof(double) * c->N));

@@ -6,7 +6,7 @@
 // owns a W x W core of nodes and loads its core plus a halo of K nodes on each side (T x T
 // nodes, T = 24..32, the side with the least rounds of the CUs times T^2) into the LDS,
 // coalesced; each of the K steps pulls from the LDS (boundary rules applied by the values the
-// live nodes write, tb_links) and collides in registers (one thread per node), and the live
+// live nodes write, setup_links9) and collides in registers (one thread per node), and the live
 // nodes write their populations back to the LDS.  A halo node's result is exact as long as every node it pulled from was, so the exact
 // region shrinks by one node per step and after K steps covers the core, which is written out;
 // each step computes only that region (threads in ring order, the waves outside it idle).  No

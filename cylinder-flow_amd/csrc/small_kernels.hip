@@ -79,34 +79,6 @@ int tb_tile(const Geo &g, int K, int cus) {
     return best;
 }
 
-std::vector<uint16_t> tb_links(const Geo &g, const std::vector<uint8_t> &flags) {
-    using L = Lat<9>;
-    std::vector<uint16_t> lk(flags.size(), 0);
-    for (int y = 0; y < g.ny; y++) {
-        const bool wallrow = !g.yper && (y == 0 || y == g.ny - 1);
-        for (int x = 0; x < g.nx; x++) {
-            const size_t node = (size_t)x + (size_t)g.nxp * y;
-            if (flags[node] == FL_SOLID || (!wallrow && flags[node] != FL_NEAR)) continue;
-            uint16_t b = 0;
-            for (int i = 1; i < 9; i++) {
-                const int ex = L::ex(i), ey = L::ey(i);
-                if (ex > 0 && x == 0 && !g.xper) continue;                 // Zou-He unknown
-                int sx = x - ex, sy = y - ey;
-                if (g.yper) sy = (sy + g.ny) % g.ny;
-                if (sy < 0 || sy >= g.ny) {                                // wall
-                    b |= (uint16_t)(1u << (7 + i));
-                    continue;
-                }
-                if (g.xper) sx = (sx + g.nx) % g.nx;
-                else if (sx == g.nx) sx = x;                               // outlet clamp
-                if (flags[(size_t)sx + (size_t)g.nxp * sy] == FL_SOLID) b |= (uint16_t)(1u << (i - 1));
-            }
-            lk[node] = b;
-        }
-    }
-    return lk;
-}
-
 // record slots of the partials buffer: the force records of several launches are summed by one
 // k_tb_force launch (a launch of its own costs about as much as a step)
 int tb_records(int K) { return K > 128 ? K : 128; }
