@@ -28,10 +28,6 @@ static int aerr(lbm_ctx *c, int code, const std::string &m) {
         }                                                                                              \
     } while (0)
 
-static double weight(int m, int n0, int n1, double scale) {
-    return (m >= n0 && m <= n1) ? scale / (double)(n1 - n0 + 1) : 0.0;
-}
-
 FusedArgs ctx_fused_args(const lbm_ctx *c);
 StepBufs step_bufs(const lbm_ctx *c, const void *A, void *B);
 
@@ -54,6 +50,7 @@ extern "C" int lbm_adjoint(lbm_ctx *c, int n0, int n1, double scale, int K, doub
     hipEvent_t e0 = nullptr, e1 = nullptr, e2 = nullptr;
     float tf = 0.f, ta = 0.f;
     const FusedArgs fa = ctx_fused_args(c);
+    const AdjWindow win{n0, n1, scale / (double)(n1 - n0 + 1)};
     const int fi_saved = c->cfg.force_interval;
     std::vector<double> hist;
     size_t freeb = 0, totalb = 0;
@@ -80,6 +77,16 @@ extern "C" int lbm_adjoint(lbm_ctx *c, int n0, int n1, double scale, int K, doub
     ATRY(hipEventCreate(&e1));
     ATRY(hipEventCreate(&e2));
 
+    if (c->tb_k >= 2) {
+        AdjSmall l{};
+        l.sfrac = c->dsfrac;
+        l.T = c->tb_t;
+        l.K = c->tb_k;
+        l.steps = 1;
+        l.prepare = true;
+        ATRY(adj_small(c->prec, l, fa, c->stream));
+    }
+
     // ---- forward with checkpoints, drag every step ----
     c->cfg.force_interval = 1;
     ATRY(hipEventRecord(e0, c->stream));
@@ -98,21 +105,44 @@ extern "C" int lbm_adjoint(lbm_ctx *c, int n0, int n1, double scale, int K, doub
             const int m0 = k * K;
             const int n = (m0 + K <= n1) ? K : n1 - m0;
             ATRY(hipMemcpyAsync(store, (char *)ckpt + SZ * k, SZ, hipMemcpyDeviceToDevice, c->stream));
-            for (int t = 0; t + 1 < n; t++)
-                ATRY(plain_step(Q, c->prec, c->V, step_bufs(c, (char *)store + SZ * t, (char *)store + SZ * (t + 1)),
-                                false, false, fa, c->stream));
-            for (int t = n - 1; t >= 0; t--) {
+            for (int t = 0; t + 1 < n;) {
+                char *const H = (char *)store + SZ * t;
+                // Small D2Q9 domains: tb_k steps per launch, every state stored (400x100 FP64: 1000 steps'
+                // recompute 3.8 -> 2.0 ms).  D3Q27 stays at one step per launch: the write of every state
+                // bounds it either way (192x96x96 FP32, two steps per pass with both states stored, 75 us
+                // per step against 67: the read a second step saves came from the last-level cache).
+                if (c->tb_k >= 2 && n - 1 - t >= 2) {
+                    int nrec = 0;
+                    const int steps = n - 1 - t < c->tb_k ? n - 1 - t : c->tb_k;
+                    ATRY(tb_steps(c->prec, H, H + SZ * steps, c->flags, c->tb_lk, c->dsfrac, c->duin, c->tb_partials, 0, &nrec, fa,
+                                  c->tb_t, c->tb_k, steps, m0 + t, 0, H + SZ, SZ / esz, c->stream));
+                    t += steps;
+                } else {
+                    ATRY(plain_step(Q, c->prec, c->V, step_bufs(c, H, H + SZ), false, false, fa, c->stream));
+                    t++;
+                }
+            }
+            for (int t = n - 1; t >= 0;) {
                 const int m = m0 + t + 1;
+                if (c->tb_k >= 2 && t >= 1) {   // the steps m, m - 1, ... of a launch
+                    const int steps = t + 1 < c->tb_k ? t + 1 : c->tb_k;
+                    ATRY(adj_small(c->prec, AdjSmall{(char *)store + SZ * t, SZ / esz, mun, mu, c->flags, c->tb_lk, c->dsfrac, c->duin,
+                                                     dJds, dJdu, win, m, c->tb_t, c->tb_k, steps, false}, fa, c->stream));
+                    std::swap(mun, mu);
+                    t -= steps;
+                    continue;
+                }
                 AdjArgs aa;
                 aa.f = fa;
-                aa.alpha = weight(m, n0, n1, scale);
-                aa.alpha_next = weight(m + 1, n0, n1, scale);
+                aa.alpha = win.at(m);
+                aa.alpha_next = win.at(m + 1);
                 ATRY(adj_step(Q, c->prec, (char *)store + SZ * t, mun, mu, c->flags, c->dsfrac, c->duin, dJds, dJdu, c->rowclean, c->adj_all_fast, aa,
                               c->stream));
                 std::swap(mun, mu);
+                t--;
             }
         }
-        ATRY(adj_init(Q, c->prec, mun, c->flags, c->duin, dxi, c->cfg.perturb, c->cfg.seed, weight(1, n0, n1, scale),
+        ATRY(adj_init(Q, c->prec, mun, c->flags, c->duin, dxi, c->cfg.perturb, c->cfg.seed, win.at(1),
                       dJdu, fa, c->stream));
     }
     ATRY(hipEventRecord(e2, c->stream));
@@ -127,7 +157,7 @@ extern "C" int lbm_adjoint(lbm_ctx *c, int n0, int n1, double scale, int K, doub
         hist.resize(4 * (size_t)c->nrec);
         ATRY(hipMemcpy(hist.data(), c->hist, sizeof(double) * hist.size(), hipMemcpyDeviceToHost));
         double acc = 0.0;
-        for (int r = 0; r < c->nrec; r++) acc += weight((int)hist[4 * r], n0, n1, scale) * hist[4 * r + 1];
+        for (int r = 0; r < c->nrec; r++) acc += win.at((int)hist[4 * r]) * hist[4 * r + 1];
         *J = acc;
     }
     if (dJ_ds) {

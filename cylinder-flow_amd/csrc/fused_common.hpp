@@ -292,4 +292,12 @@ __device__ __forceinline__ void collide_f64(const double *gv, double sf, double 
     });
 }
 
+// LDS between threads of the block, nothing else: outstanding loads and stores of global memory
+// stay in flight across it
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 }  // namespace lbm

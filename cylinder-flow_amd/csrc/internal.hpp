@@ -172,11 +172,11 @@ int tb_tile(const Geo &g, int K, int cus);
 hipError_t tb_prepare(int prec, int T, const void *sfrac, const FusedArgs &a);
 // tb_steps: `steps` (<= K) steps in one launch; the partials of its force records go to record
 // slots pend, pend + 1, ... of `partials` (tb_records() slots of ntiles * 3 doubles); *nrec = their
-// count.
+// count.  keep (null: none): the state after step k < steps of the launch goes to keep + (k - 1) * keep_stride (elements)
 int tb_records(int K);
 hipError_t tb_steps(int prec, const void *A, void *B, const uint8_t *flags, const uint16_t *lk, const void *sfrac,
                     const double *uin, double *partials, int pend, int *nrec, const FusedArgs &a, int T, int K, int steps,
-                    long step0, int fi, hipStream_t s);
+                    long step0, int fi, void *keep, size_t keep_stride, hipStream_t s);
 // sums npend record slots (of `slots`) of nparts triples each into hist[rec0 ...], the first at step step1
 hipError_t tb_force_flush(const double *partials, int nparts, int slots, double *hist, int rec0, int npend, long step1, int fi,
                           hipStream_t s);
@@ -282,6 +282,30 @@ struct AdjArgs {
 hipError_t adj_step(int Q, int prec, const void *H, const void *mu_next, void *mu, const uint8_t *flags,
                     const void *sfrac, const double *uin, void *dJds, double *dJdu_rows, const uint8_t *rowclean,
                     bool all_fast, const AdjArgs &a, hipStream_t s);
+// weight of step m: w within n0 .. n1, else 0
+struct AdjWindow {
+    int n0, n1;
+    double w;
+    __host__ __device__ double at(int m) const { return m >= n0 && m <= n1 ? w : 0.0; }
+};
+// several reverse steps per launch on small non-periodic D2Q9 domains (adjoint_small.hip): steps m, m - 1, ...
+// (steps <= K of them) from mun = mu_{m+1} to mu; H: H_{m-1}, H_{m-2} `stride` elements below it and so on;
+// tiles as tb_steps
+struct AdjSmall {
+    const void *H;
+    size_t stride;
+    const void *mun;
+    void *mu;
+    const uint8_t *flags;
+    const uint16_t *lk;
+    const void *sfrac;
+    const double *uin;
+    double *dJds, *dJdu;
+    AdjWindow win;
+    int m, T, K, steps;
+    bool prepare;   // only set the kernel's LDS limit on the current device
+};
+hipError_t adj_small(int prec, const AdjSmall &l, const FusedArgs &a, hipStream_t s);
 hipError_t adj_init(int Q, int prec, const void *mu1, const uint8_t *flags, const double *uin,
                     const double *xi, double perturb, uint64_t seed, double alpha1, double *dJdu_rows,
                     const FusedArgs &a, hipStream_t s);

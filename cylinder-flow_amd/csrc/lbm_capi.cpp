@@ -913,7 +913,7 @@ static int step_n(lbm_ctx *c, int n, hipEvent_t *evs = nullptr) {
             HIP_TRY(c, strip_launch(c->prec, l, a, c->stream));
         } else {
             HIP_TRY(c, tb_steps(c->prec, c->A, c->B, c->flags, c->tb_lk, c->dsfrac, c->duin, c->tb_partials, pend, &nr, a, c->tb_t,
-                                c->tb_k, kk, c->step, fi, c->stream));
+                                c->tb_k, kk, c->step, fi, nullptr, 0, c->stream));
         }
         pend += nr;
         c->nrec += nr;

@@ -16,7 +16,7 @@
 // The loads of plane k + 1 are issued before the arithmetic of plane k and stay in flight behind
 // it.  The rim is computed by every block that needs it (no block waits for another).
 //
-// Half-way bounce-back (walls and mask links) comes from a word per node computed on the host:
+// Half-way bounce-back (walls and mask links) comes from a word per node (pair_words.hip):
 // bit i, direction i takes the node's own h_opp(i).  Blocks read the words only of planes where
 // the column or its rim holds one (a bit per column and plane), and only waves that hold one do
 // more than the plain pull; elsewhere the pull has no rule but the x edges: the inlet's unknowns are overwritten by the inlet rule, the outlet's source is
@@ -129,14 +129,6 @@ __device__ __forceinline__ V pair_pick(uint32_t w, int i, V a, V b) {
         __builtin_memcpy(&r, &x, sizeof(V));
     }
     return r;
-}
-
-// LDS between threads of the block, nothing else: outstanding loads and stores of global memory
-// stay in flight across it
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
 // LDS of a block: one plane of stored values, then the column's own bounced values (see k_pair)

@@ -26,52 +26,19 @@ constexpr int TB_KMAX = 10;   // steps per launch at most (tb_depth)
 // LDS row length (doubles) of a T x T tile: the odd one of T + 1, T + 2
 __host__ __device__ constexpr int tb_row(int T) { return T % 2 == 0 ? T + 1 : T + 2; }
 
-template <class S, int TB_T, bool ANY_FORCE, bool SFRAC>
-__global__ void __launch_bounds__(1024)
-    k_tb2d(const typename S::T *__restrict__ A, typename S::T *__restrict__ B, const uint8_t *__restrict__ flags,
-           const uint16_t *__restrict__ lk, const typename S::C *__restrict__ sfrac, const double *__restrict__ uin,
-           double *__restrict__ partials,
-           const FusedArgs a, int K, int steps, long step0, int fi, int tiles_x, int ntiles, int pend) {
-    using L = Lat<9>;
-    using T = typename S::T;
-    using C = typename S::C;
-    // one thread per node of the rings a step can compute (within K - 1 of the core); the
-    // outermost ring is only read, and is loaded with the rest of the tile
-    constexpr int Q = 9, NT = (TB_T - 2) * (TB_T - 2);
-    static_assert((NT + 63) / 64 <= 16, "force records hold 16 waves");
-    const Geo &g = a.g;
-    const int W = TB_T - 2 * K;          // core side
-    // LDS: two halves of Q x TB_T x TP values (step s reads half s % 2; node (tx, ty) at
-    // tx * TP + ty, rows padded to the odd TP = tb_row(TB_T) so that lanes TP apart hit different
-    // banks: an even row of 32 doubles puts every x of a row segment on one bank),
-    // then the tile's link words (TB_T x TP) and flags (TB_T x TP bytes)
-    constexpr int TP = tb_row(TB_T), HALF = Q * TB_T * TP;
-    extern __shared__ __align__(16) char tb_lds[];
-    T *const lds = (T *)tb_lds;
-    uint16_t *llk = (uint16_t *)(lds + 2 * HALF);
-    uint8_t *lfl = (uint8_t *)(llk + TB_T * TP);
-    // Threads take the tile's nodes ring by ring from the core outwards: threads [0, W*W) the
-    // core (y fastest), then ring r = 1..K-1 (the nodes at Chebyshev distance r from the core:
-    // its left and right columns, then its top and bottom rows).  The nodes a step must compute,
-    // the live nodes within the steps still to come of the core, are then the first (W + 2m)^2
-    // threads, and the waves beyond them skip the step: the busiest SIMD of a 24 x 24 tile runs
-    // 2+2+2+1+1 wave-steps in 5 steps instead of 3 per step.  Tiles at the inlet (their left K
-    // columns lie outside the domain) take the inlet column x = 0 first, so that one wave runs
-    // the inlet's long sequence, then the nodes right of it ring by ring, then those left of it
-    // (never computed).
-    const int t = threadIdx.x;
-    // Workgroups go to the 8 XCDs in turn (b % 8), each XCD with its own L2: XCD k takes the
-    // consecutive positions [k (n / 8) + min(k, n % 8), ...) of the n = ntiles in an order that
-    // runs down bands of two tile rows column by column, so that an XCD holds a 2-row block of
-    // neighbouring tiles, whose loads overlap, read through one L2 (on 400 x 100, 2 x 14-15
-    // tiles per XCD: 10 % fewer microseconds per step than neighbouring tiles on different XCDs)
-    const int xcd = (int)(blockIdx.x % 8u);
-    const int pos = xcd * (ntiles / 8) + min(xcd, ntiles % 8) + (int)(blockIdx.x / 8u);
-    const int band = pos / (2 * tiles_x), in_band = pos % (2 * tiles_x);
-    const int band_rows = min(2, ntiles / tiles_x - 2 * band);
-    const int tile = (2 * band + in_band % band_rows) * tiles_x + in_band / band_rows;
-    int tx, ty;
-    if (tile % tiles_x != 0) {
+// Threads take the tile's nodes ring by ring from the core outwards: threads [0, W*W) the
+// core (y fastest), then ring r = 1..K-1 (the nodes at Chebyshev distance r from the core:
+// its left and right columns, then its top and bottom rows).  The nodes a step must compute,
+// the live nodes within the steps still to come of the core, are then the first (W + 2m)^2
+// threads, and the waves beyond them skip the step: the busiest SIMD of a 24 x 24 tile runs
+// 2+2+2+1+1 wave-steps in 5 steps instead of 3 per step.  Tiles at the inlet (their left K
+// columns lie outside the domain) take the inlet column x = 0 first, so that one wave runs
+// the inlet's long sequence, then the nodes right of it ring by ring, then those left of it
+// (never computed).
+template <int TB_T>
+__device__ __forceinline__ void tb_place(int t, int K, bool inlet, int &tx, int &ty) {
+    const int W = TB_T - 2 * K;
+    if (!inlet) {
         if (t < W * W) {
             tx = K + t / W;
             ty = K + t % W;
@@ -128,6 +95,49 @@ __global__ void __launch_bounds__(1024)
             }
         }
     }
+}
+
+// Workgroups go to the 8 XCDs in turn (b % 8), each XCD with its own L2: XCD k takes the
+// consecutive positions [k (n / 8) + min(k, n % 8), ...) of the n = ntiles in an order that
+// runs down bands of two tile rows column by column, so that an XCD holds a 2-row block of
+// neighbouring tiles, whose loads overlap, read through one L2 (on 400 x 100, 2 x 14-15
+// tiles per XCD: 10 % fewer microseconds per step than neighbouring tiles on different XCDs)
+__device__ __forceinline__ int tb_tile_of_block(int tiles_x, int ntiles) {
+    const int xcd = (int)(blockIdx.x % 8u);
+    const int pos = xcd * (ntiles / 8) + min(xcd, ntiles % 8) + (int)(blockIdx.x / 8u);
+    const int band = pos / (2 * tiles_x), in_band = pos % (2 * tiles_x);
+    const int band_rows = min(2, ntiles / tiles_x - 2 * band);
+    return (2 * band + in_band % band_rows) * tiles_x + in_band / band_rows;
+}
+
+template <class S, int TB_T, bool ANY_FORCE, bool SFRAC>
+__global__ void __launch_bounds__(1024)
+    k_tb2d(const typename S::T *__restrict__ A, typename S::T *__restrict__ B, const uint8_t *__restrict__ flags,
+           const uint16_t *__restrict__ lk, const typename S::C *__restrict__ sfrac, const double *__restrict__ uin,
+           double *__restrict__ partials, typename S::T *__restrict__ keep, size_t keep_stride,
+           const FusedArgs a, int K, int steps, long step0, int fi, int tiles_x, int ntiles, int pend) {
+    using L = Lat<9>;
+    using T = typename S::T;
+    using C = typename S::C;
+    // one thread per node of the rings a step can compute (within K - 1 of the core); the
+    // outermost ring is only read, and is loaded with the rest of the tile
+    constexpr int Q = 9, NT = (TB_T - 2) * (TB_T - 2);
+    static_assert((NT + 63) / 64 <= 16, "force records hold 16 waves");
+    const Geo &g = a.g;
+    const int W = TB_T - 2 * K;          // core side
+    // LDS: two halves of Q x TB_T x TP values (step s reads half s % 2; node (tx, ty) at
+    // tx * TP + ty, rows padded to the odd TP = tb_row(TB_T) so that lanes TP apart hit different
+    // banks: an even row of 32 doubles puts every x of a row segment on one bank),
+    // then the tile's link words (TB_T x TP) and flags (TB_T x TP bytes)
+    constexpr int TP = tb_row(TB_T), HALF = Q * TB_T * TP;
+    extern __shared__ __align__(16) char tb_lds[];
+    T *const lds = (T *)tb_lds;
+    uint16_t *llk = (uint16_t *)(lds + 2 * HALF);
+    uint8_t *lfl = (uint8_t *)(llk + TB_T * TP);
+    const int t = threadIdx.x;
+    const int tile = tb_tile_of_block(tiles_x, ntiles);
+    int tx, ty;
+    tb_place<TB_T>(t, K, tile % tiles_x == 0, tx, ty);
     // Chebyshev distance of the node from the core
     const int dx = tx < K ? K - tx : (tx >= K + W ? tx - (K + W - 1) : 0);
     const int dy = ty < K ? K - ty : (ty >= K + W ? ty - (K + W - 1) : 0);
@@ -212,6 +222,15 @@ __global__ void __launch_bounds__(1024)
     // launch's last barrier, so no force step waits for a block-wide sum
     __shared__ double red[3 * 16 * TB_KMAX];
     int sf = ANY_FORCE && fi > 0 ? (int)(fi - 1 - step0 % fi) : -1, kr = 0;
+    auto store_core = [&](const T *from, T *to) {   // x fastest
+        for (int j = t; j < W * W; j += NT) {
+            const int lx = K + j % W, ly = K + j / W, AX = X0 + lx, AY = Y0 + ly;
+            if (AX < g.nx && AY < g.ny && lfl[lx * TP + ly] != FL_SOLID)
+                static_for<0, Q>([&](auto I) {
+                    __builtin_nontemporal_store(from[I * TB_T * TP + lx * TP + ly], &to[pel(g, I, (uint32_t)AX, (uint32_t)AY)]);
+                });
+        }
+    };
     for (int s = 0; s < steps; s++) {
         const bool force = ANY_FORCE && s == sf;
         // two halves: the barrier of step s also orders the reads of step s - 1 before the writes
@@ -237,6 +256,7 @@ __global__ void __launch_bounds__(1024)
                     });
             }
             __syncthreads();
+            if (keep != nullptr) store_core(buf, keep + keep_stride * (size_t)(s - 1));
         }
         double fx = 0.0, fy = 0.0;
         if (dist <= rs && live) {
@@ -305,13 +325,7 @@ __global__ void __launch_bounds__(1024)
         P[1] = fy;
         P[2] = fz;
     }
-    for (int j = t; j < W * W; j += NT) {
-        const int lx = K + j % W, ly = K + j / W, AX = X0 + lx, AY = Y0 + ly;
-        if (AX < g.nx && AY < g.ny && lfl[lx * TP + ly] != FL_SOLID)
-            static_for<0, Q>([&](auto I) {
-                __builtin_nontemporal_store(out[I * TB_T * TP + lx * TP + ly], &B[pel(g, I, (uint32_t)AX, (uint32_t)AY)]);
-            });
-    }
+    store_core(out, B);
 }
 
 // ---- launchers of one storage format (small_f64.hip ... small_bf16.hip) ----
@@ -327,6 +341,8 @@ struct TbLaunch {
     const void *sfrac;
     const double *uin;
     double *partials;
+    void *keep;            // null, or where the states before the last go, keep_stride elements apart
+    size_t keep_stride;
     int T, K, steps, fi, tiles_x, ntiles, pend;
     long step0;
     bool force;
@@ -368,7 +384,7 @@ static hipError_t tb_launch_s(const TbLaunch &l, const FusedArgs &a, hipStream_t
                 return;
             }
             hipLaunchKernelGGL(kern, dim3(l.ntiles), dim3((W - 2) * (W - 2)), lds, s, (const T *)l.A, (T *)l.B, l.flags, l.lk,
-                               (const typename S::C *)l.sfrac, l.uin, l.partials, a, l.K, l.steps, l.step0, l.fi, l.tiles_x,
+                               (const typename S::C *)l.sfrac, l.uin, l.partials, (T *)l.keep, l.keep_stride, a, l.K, l.steps, l.step0, l.fi, l.tiles_x,
                                l.ntiles, l.pend);
             e = hipGetLastError();
         };

@@ -108,15 +108,15 @@ hipError_t tb_prepare(int prec, int T, const void *sfrac, const FusedArgs &a) {
 // tb_records(K) and sums them with tb_force_flush).  Returns the number of records.
 hipError_t tb_steps(int prec, const void *A, void *B, const uint8_t *flags, const uint16_t *lk, const void *sfrac,
                     const double *uin, double *partials, int pend, int *nrec, const FusedArgs &a, int T, int K, int steps,
-                    long step0, int fi, hipStream_t s) {
+                    long step0, int fi, void *keep, size_t keep_stride, hipStream_t s) {
     int tiles_x = 0;
     const int ntiles = tb_tiles(a.g, T, K, &tiles_x);
     const int nforce = fi > 0 ? (int)((step0 + steps) / fi - step0 / fi) : 0;
     *nrec = nforce;
     if (pend < 0 || pend + nforce > tb_records(K)) return hipErrorInvalidValue;
     if (T - 2 * K < 1 || K > TB_KMAX || steps < 1 || steps > K) return hipErrorInvalidValue;
-    return tb_launch(prec, TbLaunch{A, B, flags, lk, sfrac, uin, partials, T, K, steps, fi, tiles_x, ntiles, pend, step0,
-                                    nforce > 0, false}, a, s);
+    return tb_launch(prec, TbLaunch{A, B, flags, lk, sfrac, uin, partials, keep, keep_stride, T, K, steps, fi, tiles_x, ntiles, pend,
+                                    step0, nforce > 0, false}, a, s);
 }
 
 hipError_t tb_force_flush(const double *partials, int nparts, int slots, double *hist, int rec0, int npend, long step1, int fi,
