@@ -39,10 +39,22 @@ extern "C" int lbm_adjoint(lbm_ctx *c, int n0, int n1, double scale, int K, doub
     if (!c->initialized || c->step != 0) return aerr(c, LBM_ERR_STATE, "lbm_adjoint needs a freshly initialised context (step 0)");
     if (n0 < 1 || n1 < n0) return aerr(c, LBM_ERR_INVALID, "need 1 <= n0 <= n1");
     if (K <= 0 || K > n1) K = n1;
+    const int K_asked = K;
     const Geo &g = c->geo;
     const int Q = c->Q;
     const size_t esz = c->prec == LBM_FP64 ? 8 : 4;
     const size_t SZ = esz * Q * g.plane;
+    // Freed device memory is cleared before it is given out again, at about 40 GB/s behind the program's
+    // back: a program that evaluates gradients one after another runs into that once it has gone through
+    // the card's memory, and then pays for every byte of the store (192x96x96 FP32, 400 steps, K = 50, 11.4 GB
+    // per evaluation: 295 ms on average over 80 evaluations, 115 for each of the first 24).  From 4 GB on the
+    // segments are therefore no longer than sqrt(n1) steps, the split with the least states, at the same
+    // recompute; below, what is freed is cleared during the next evaluation, and longer segments leave
+    // fewer remainders of the steps per launch.
+    if ((double)SZ * ((n1 + K - 1) / K + K) >= 4e9) {
+        const int root = (int)std::ceil(std::sqrt((double)n1));
+        if (root < K) K = root;
+    }
     const int nseg = (n1 + K - 1) / K;
     int rc = LBM_OK;
     void *ckpt = nullptr, *store = nullptr, *mu0 = nullptr, *mu1 = nullptr;
@@ -56,11 +68,13 @@ extern "C" int lbm_adjoint(lbm_ctx *c, int n0, int n1, double scale, int K, doub
     size_t freeb = 0, totalb = 0;
 
     (void)hipMemGetInfo(&freeb, &totalb);
-    if ((double)SZ * (nseg + K + 2) + 8.0 * g.plane * 2 > 0.95 * (double)freeb)
-        return aerr(c, LBM_ERR_NOMEM, "adjoint store (" + std::to_string((double)SZ * (nseg + K + 2) / 1e9) +
+    // (the store of the segments asked for: what was refused does not depend on the split above)
+    const int asked = (n1 + K_asked - 1) / K_asked + K_asked + 2;
+    if ((double)SZ * asked + 8.0 * g.plane * 2 > 0.95 * (double)freeb)
+        return aerr(c, LBM_ERR_NOMEM, "adjoint store (" + std::to_string((double)SZ * asked / 1e9) +
                                          " GB) exceeds free device memory; lower checkpoint_every");
     ATRY(hipMalloc(&ckpt, SZ * nseg));
-    ATRY(hipMalloc(&store, SZ * K));
+    if (K > 1) ATRY(hipMalloc(&store, SZ * (K - 1)));   // a segment's states but its first, which is the checkpoint
     ATRY(hipMalloc(&mu0, SZ));
     ATRY(hipMalloc(&mu1, SZ));
     ATRY(hipMalloc(&dJds, sizeof(double) * g.plane));
@@ -104,9 +118,9 @@ extern "C" int lbm_adjoint(lbm_ctx *c, int n0, int n1, double scale, int K, doub
         for (int k = nseg - 1; k >= 0; k--) {
             const int m0 = k * K;
             const int n = (m0 + K <= n1) ? K : n1 - m0;
-            ATRY(hipMemcpyAsync(store, (char *)ckpt + SZ * k, SZ, hipMemcpyDeviceToDevice, c->stream));
+            auto state = [&](int t) { return t == 0 ? (char *)ckpt + SZ * k : (char *)store + SZ * (t - 1); };
             for (int t = 0; t + 1 < n;) {
-                char *const H = (char *)store + SZ * t;
+                char *const H = state(t), *const next = state(t + 1);
                 // Small D2Q9 domains: tb_k steps per launch, every state stored (400x100 FP64: 1000 steps'
                 // recompute 3.8 -> 2.0 ms).  D3Q27 stays at one step per launch: the write of every state
                 // bounds it either way (192x96x96 FP32, two steps per pass with both states stored, 75 us
@@ -114,11 +128,11 @@ extern "C" int lbm_adjoint(lbm_ctx *c, int n0, int n1, double scale, int K, doub
                 if (c->tb_k >= 2 && n - 1 - t >= 2) {
                     int nrec = 0;
                     const int steps = n - 1 - t < c->tb_k ? n - 1 - t : c->tb_k;
-                    ATRY(tb_steps(c->prec, H, H + SZ * steps, c->flags, c->tb_lk, c->dsfrac, c->duin, c->tb_partials, 0, &nrec, fa,
-                                  c->tb_t, c->tb_k, steps, m0 + t, 0, H + SZ, SZ / esz, c->stream));
+                    ATRY(tb_steps(c->prec, H, next + SZ * (steps - 1), c->flags, c->tb_lk, c->dsfrac, c->duin, c->tb_partials, 0, &nrec, fa,
+                                  c->tb_t, c->tb_k, steps, m0 + t, 0, next, SZ / esz, c->stream));
                     t += steps;
                 } else {
-                    ATRY(plain_step(Q, c->prec, c->V, step_bufs(c, H, H + SZ), false, false, fa, c->stream));
+                    ATRY(plain_step(Q, c->prec, c->V, step_bufs(c, H, next), false, false, fa, c->stream));
                     t++;
                 }
             }
@@ -126,7 +140,7 @@ extern "C" int lbm_adjoint(lbm_ctx *c, int n0, int n1, double scale, int K, doub
                 const int m = m0 + t + 1;
                 if (c->tb_k >= 2 && t >= 1) {   // the steps m, m - 1, ... of a launch
                     const int steps = t + 1 < c->tb_k ? t + 1 : c->tb_k;
-                    ATRY(adj_small(c->prec, AdjSmall{(char *)store + SZ * t, SZ / esz, mun, mu, c->flags, c->tb_lk, c->dsfrac, c->duin,
+                    ATRY(adj_small(c->prec, AdjSmall{state(t), state(t - steps + 1), SZ / esz, mun, mu, c->flags, c->tb_lk, c->dsfrac, c->duin,
                                                      dJds, dJdu, win, m, c->tb_t, c->tb_k, steps, false}, fa, c->stream));
                     std::swap(mun, mu);
                     t -= steps;
@@ -136,7 +150,7 @@ extern "C" int lbm_adjoint(lbm_ctx *c, int n0, int n1, double scale, int K, doub
                 aa.f = fa;
                 aa.alpha = win.at(m);
                 aa.alpha_next = win.at(m + 1);
-                ATRY(adj_step(Q, c->prec, (char *)store + SZ * t, mun, mu, c->flags, c->dsfrac, c->duin, dJds, dJdu, c->rowclean, c->adj_all_fast, aa,
+                ATRY(adj_step(Q, c->prec, state(t), mun, mu, c->flags, c->dsfrac, c->duin, dJds, dJdu, c->rowclean, c->adj_all_fast, aa,
                               c->stream));
                 std::swap(mun, mu);
                 t--;

@@ -16,7 +16,7 @@ namespace lbm {
 
 template <class S, int TB_T, bool SFRAC>
 __global__ void __launch_bounds__((TB_T - 2) * (TB_T - 2))
-    k_adj2d(const typename S::T *__restrict__ H, size_t stride, const typename S::C *__restrict__ mun,
+    k_adj2d(const typename S::T *__restrict__ H, const typename S::T *__restrict__ Hlast, size_t stride, const typename S::C *__restrict__ mun,
             typename S::C *__restrict__ mu, const uint8_t *__restrict__ flags, const uint16_t *__restrict__ lk,
             const typename S::C *__restrict__ sfrac, const double *__restrict__ uin, double *__restrict__ dJds,
             double *__restrict__ dJdu, const FusedArgs a, AdjWindow win, int m, int K, int steps, int tiles_x, int ntiles) {
@@ -82,7 +82,7 @@ __global__ void __launch_bounds__((TB_T - 2) * (TB_T - 2))
         });
     }
     T rh[Q] = {};
-    if (dist <= steps - 1) static_for<0, Q>([&](auto I) { rh[I] = H[off[I]]; });
+    if (dist <= steps - 1) static_for<0, Q>([&](auto I) { rh[I] = H[off[I]]; });   // (steps == 1: H is Hlast)
     C mm[Q] = {};
     for (int s = 0; s < steps; s++, m--) {
         lds_barrier();
@@ -96,7 +96,7 @@ __global__ void __launch_bounds__((TB_T - 2) * (TB_T - 2))
             if constexpr (L::ex(i) > 0) gv[i] = xlo ? (C)0 : gv[i];
         });
         if (dist < rs) {   // the next step's
-            const T *const Hn = H - stride * (size_t)(s + 1);
+            const T *const Hn = s + 2 == steps ? Hlast : H - stride * (size_t)(s + 1);
             static_for<0, Q>([&](auto I) { rh[I] = Hn[off[I]]; });
         }
         if (dist <= rs) {
@@ -157,7 +157,7 @@ static hipError_t adj_small_s(const AdjSmall &l, const FusedArgs &a, hipStream_t
                 e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
                 return;
             }
-            hipLaunchKernelGGL(kern, dim3((unsigned)ntiles), dim3((W - 2) * (W - 2)), lds, s, (const T *)l.H, l.stride,
+            hipLaunchKernelGGL(kern, dim3((unsigned)ntiles), dim3((W - 2) * (W - 2)), lds, s, (const T *)l.H, (const T *)l.Hlast, l.stride,
                                (const C *)l.mun, (C *)l.mu, l.flags, l.lk, (const C *)l.sfrac, l.uin, l.dJds, l.dJdu, a, l.win, l.m,
                                l.K, l.steps, tiles_x, ntiles);
             e = hipGetLastError();

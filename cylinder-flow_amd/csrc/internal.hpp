@@ -289,10 +289,10 @@ struct AdjWindow {
     __host__ __device__ double at(int m) const { return m >= n0 && m <= n1 ? w : 0.0; }
 };
 // several reverse steps per launch on small non-periodic D2Q9 domains (adjoint_small.hip): steps m, m - 1, ...
-// (steps <= K of them) from mun = mu_{m+1} to mu; H: H_{m-1}, H_{m-2} `stride` elements below it and so on;
-// tiles as tb_steps
+// (steps <= K of them) from mun = mu_{m+1} to mu; H: H_{m-1}, the states before it `stride` elements apart
+// below it, but for the last of the launch, which is Hlast; tiles as tb_steps
 struct AdjSmall {
-    const void *H;
+    const void *H, *Hlast;
     size_t stride;
     const void *mun;
     void *mu;
