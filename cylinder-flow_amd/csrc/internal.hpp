@@ -143,7 +143,7 @@ struct PairPlan {
     uint32_t *fblk = nullptr;     // the blocks in slot order (null: per node)
     int fbx = 0, fgx = 0;
     int nslots = 0;
-    double *partials = nullptr;   // the slots, then their chunk sums
+    double *partials = nullptr;   // force_bytes(nslots)
 };
 struct PairOps {   // a storage format's column, LDS bytes and launchers
     int wx, wy;
@@ -198,10 +198,12 @@ hipError_t strip_launch(int prec, const StripLaunch &l, const FusedArgs &a, hipS
 // fills steps, strips, rows and nwaves
 void strip_shape(const Geo &g, int prec, int cus, int steps, StripLaunch &l);
 
-// sum of the nslots force partials into hist[rec] (chunks: force_chunks(nslots) * 3 doubles)
-int force_chunks(int nslots);
-hipError_t force_reduce(const double *partials, int nslots, double *chunks, double *hist, int rec, long step,
-                        hipStream_t s);
+// force partials: a buffer of force_bytes(nslots) keeps those of force_records(nslots) steps, 3 * nslots
+// doubles each; force_reduce sums the first nrec of them into hist[rec], hist[rec + 1], ... (steps step,
+// step + every, ...)
+int force_records(int nslots);
+size_t force_bytes(int nslots);
+hipError_t force_reduce(double *partials, int nslots, int nrec, double *hist, int rec, long step, int every, hipStream_t s);
 // FP64 <-> storage conversion of one direction's populations (physical nodes, x fastest)
 hipError_t plain_decode(int Q, int prec, const void *A, double *out, const uint8_t *flags, int dir,
                         const FusedArgs &a, hipStream_t s);

@@ -663,7 +663,7 @@ static int init_plain(lbm_ctx *c) {
     HIP_TRY(c, hipMalloc(&c->duin, sizeof(double) * c->uin.size()));
     HIP_TRY(c, hipMalloc(&c->macros, sizeof(double) * 4 * g.plane));
     HIP_TRY(c, hipMalloc(&c->block_slot, sizeof(int) * std::max<size_t>(slot.size(), 1)));
-    HIP_TRY(c, hipMalloc(&c->partials, sizeof(double) * 3 * (std::max(c->nslots, 1) + force_chunks(c->nslots))));
+    HIP_TRY(c, hipMalloc(&c->partials, force_bytes(c->nslots)));
     // D3Q27: two steps per pass over memory where the two-step kernel applies (pair.cpp); its force
     // slots are those of the one-step path
     if (Q == 27) {
@@ -924,6 +924,34 @@ static int step_n(lbm_ctx *c, int n, hipEvent_t *evs = nullptr) {
         c->replay_ok = false;
     }
     HIP_TRY(c, tb_force_flush(c->tb_partials, nparts, slots, c->hist, rec0, pend, step1, fi, c->stream));
+    // records whose partials wait for one sum: of the two-step launches or of the one-step ones
+    struct {
+        bool pair = false;
+        int n = 0, rec0 = 0;
+        long step1 = 0;
+    } wait;
+    auto sum_waiting = [&]() {
+        const int k = wait.n;
+        wait.n = 0;
+        return force_reduce(wait.pair ? c->pair.partials : c->partials, wait.pair ? c->pair.nslots : c->nslots, k, c->hist, wait.rec0,
+                            wait.step1, fi, c->stream);
+    };
+    // the partials of the record of step `step`
+    auto next_record = [&](bool pair, long step, double *&out) {
+        const int nslots = pair ? c->pair.nslots : c->nslots;
+        if (wait.n > 0 && (wait.pair != pair || wait.n == force_records(nslots))) {
+            const hipError_t e = sum_waiting();
+            if (e != hipSuccess) return e;
+        }
+        if (wait.n == 0) {
+            wait.pair = pair;
+            wait.rec0 = c->nrec;
+            wait.step1 = step;
+        }
+        out = (pair ? c->pair.partials : c->partials) + 3 * (size_t)nslots * wait.n++;
+        c->nrec++;
+        return hipSuccess;
+    };
     while (left > 0) {
         // two steps in one pass unless the second records the force (its input stays in the LDS), or
         // the first does and a solid fraction carries force (its moments do too); not under
@@ -931,9 +959,9 @@ static int step_n(lbm_ctx *c, int n, hipEvent_t *evs = nullptr) {
         if (c->pair.on && !evs && left > 1 && !records(c->step + 2) && !(records(c->step + 1) && c->dsfrac)) {
             const PairOps ops = pair_ops(c->prec);
             if (records(c->step + 1)) {
-                HIP_TRY(c, ops.force(c->pair, c->A, c->pair.partials, a, c->stream));
-                HIP_TRY(c, force_reduce(c->pair.partials, c->pair.nslots, c->pair.partials + 3 * (size_t)c->pair.nslots, c->hist,
-                                        c->nrec++, c->step + 1, c->stream));
+                double *partials = nullptr;
+                HIP_TRY(c, next_record(true, c->step + 1, partials));
+                HIP_TRY(c, ops.force(c->pair, c->A, partials, a, c->stream));
             }
             HIP_TRY(c, ops.step(c->pair, c->A, c->B, c->dsfrac, c->duin, c->macros, false, a, c->stream));
             c->step += 2;
@@ -952,13 +980,14 @@ static int step_n(lbm_ctx *c, int n, hipEvent_t *evs = nullptr) {
             b.ev_bulk[0] = evs[2 * k];
             b.ev_bulk[1] = evs[2 * k + 1];
         }
+        if (force) HIP_TRY(c, next_record(false, c->step, b.partials));
         HIP_TRY(c, plain_step(c->Q, c->prec, c->V, b, force, false, a, c->stream));
-        if (force) HIP_TRY(c, force_reduce(c->partials, c->nslots, c->partials + 3 * (size_t)c->nslots, c->hist, c->nrec++, c->step, c->stream));
         std::swap(c->A, c->B);
         c->fields_fresh = false;
         c->replay_ok = true;
         c->replay_pair = false;
     }
+    HIP_TRY(c, sum_waiting());
     return LBM_OK;
 }
 

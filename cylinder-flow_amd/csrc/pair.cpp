@@ -92,7 +92,7 @@ hipError_t pair_plan(PairPlan &p, int prec, const Geo &g, const uint8_t *flags, 
         if (e == hipSuccess) e = hipMalloc(&p.linklk, sizeof(uint32_t) * (size_t)p.nlink);
     }
     if (e == hipSuccess) e = pair_words(p, ops, flags, g, s);
-    if (e == hipSuccess) e = hipMalloc(&p.partials, sizeof(double) * 3 * (size_t)(std::max(p.nslots, 1) + force_chunks(p.nslots)));
+    if (e == hipSuccess) e = hipMalloc(&p.partials, force_bytes(p.nslots));
     if (e != hipSuccess) {
         pair_free(p);
         if (e != hipErrorOutOfMemory) return e;
