@@ -75,8 +75,8 @@ hipError_t setup_flags(int Q, uint8_t *flags, const uint8_t *mask, const double 
                        const Geo &g, unsigned *counts, hipStream_t s);
 // per block of shape blk: 1 when it holds a node whose links or solid fraction carry force
 hipError_t setup_forced(const uint8_t *flags, const double *sfrac, uint8_t *out, Shape blk, const Geo &g, hipStream_t s);
-// per row: 1 when all its nodes are FL_FLUID
-hipError_t setup_clean(const uint8_t *flags, uint8_t *clean, const Geo &g, hipStream_t s);
+// per row: 1 when all its nodes are FL_FLUID, to both arrays
+hipError_t setup_clean(const uint8_t *flags, uint8_t *clean, uint8_t *copy, const Geo &g, hipStream_t s);
 // the solid fraction in the padded layout and the precision of the collision, 0 in the padding
 hipError_t setup_sfrac(int prec, const double *in, void *out, const Geo &g, hipStream_t s);
 // bounce-back links of the nodes for k_tb2d and k_strip: bit i-1 when direction i pulls from a solid node

@@ -423,62 +423,56 @@ static int init_plain(lbm_ctx *c) {
     // node flags, solid fraction and the counts on the device (setup_kernels.hip): from the body formula
     // (the reference's "usr", 3D MPI+KOKKOS+MPIIO/lbm.cpp:238) or the user mask
     HIP_TRY(c, hipMalloc(&c->flags, g.plane));
-    unsigned counts[3] = {0, 0, 0};      // solid, near nodes, nodes of the fix list
-    std::vector<uint8_t> forced_blk;     // per block of shape s1: holds a forced node
     const Shape s1 = c->prec == LBM_FP64 ? fp64_shape(g, Q) : lane_shape(g, 1);
-    bool per_block = c->prec == LBM_FP64;
+    // one scratch buffer; what the host reads of it comes back in one copy
+    struct Counts {
+        unsigned solid, near, fix;   // nodes of each kind, nodes of the fix list
+    } counts;
+    const size_t nblk = (size_t)s1.gx * g.ny * g.nz, nrow = (size_t)g.ny * g.nz, hold = sizeof(Counts) + nblk + nrow;
+    std::vector<uint8_t> got(hold);
     {
-        DevTmp mask, frac, cnt, blk;
-        if (c->cfg.body == LBM_BODY_MASK) {
-            HIP_TRY(c, mask.alloc(c->N));
-            HIP_TRY(c, hipMemcpyAsync(mask.p, c->solid.data(), c->N, hipMemcpyHostToDevice, c->stream));
-        }
+        const size_t fracb = sf ? sizeof(double) * c->N : 0, maskb = c->cfg.body == LBM_BODY_MASK ? c->N : 0;
+        DevTmp tmp;   // solid fraction, counts, force blocks, clean rows, mask
+        HIP_TRY(c, tmp.alloc(fracb + hold + maskb));
+        double *const frac = sf ? (double *)tmp.p : nullptr;
+        uint8_t *const res = (uint8_t *)tmp.p + fracb, *const mask = maskb ? res + hold : nullptr;
+        if (mask) HIP_TRY(c, hipMemcpyAsync(mask, c->solid.data(), c->N, hipMemcpyHostToDevice, c->stream));
         if (sf) {
-            HIP_TRY(c, frac.alloc(sizeof(double) * c->N));
-            HIP_TRY(c, hipMemcpyAsync(frac.p, c->sfrac.data(), sizeof(double) * c->N, hipMemcpyHostToDevice, c->stream));
+            HIP_TRY(c, hipMemcpyAsync(frac, c->sfrac.data(), sizeof(double) * c->N, hipMemcpyHostToDevice, c->stream));
             HIP_TRY(c, hipMalloc(&c->dsfrac, (c->prec == LBM_FP64 ? sizeof(double) : sizeof(float)) * g.plane));
-            HIP_TRY(c, setup_sfrac(c->prec, (const double *)frac.p, c->dsfrac, g, c->stream));
+            HIP_TRY(c, setup_sfrac(c->prec, frac, c->dsfrac, g, c->stream));
         }
-        HIP_TRY(c, cnt.alloc(sizeof(counts)));
+        HIP_TRY(c, hipMalloc(&c->rowclean, nrow));
         const SetupBody body{c->cfg.body, c->cfg.cx, c->cfg.cy, c->cfg.cz, c->cfg.r2};
         const SetupFix fx{V, all_slow, same_offsets};
-        HIP_TRY(c, setup_flags(Q, c->flags, (const uint8_t *)mask.p, (const double *)frac.p, body, fx, g, (unsigned *)cnt.p, c->stream));
-        HIP_TRY(c, hipMemcpyAsync(counts, cnt.p, sizeof(counts), hipMemcpyDeviceToHost, c->stream));
+        HIP_TRY(c, setup_flags(Q, c->flags, mask, frac, body, fx, g, (unsigned *)res, c->stream));
+        HIP_TRY(c, setup_forced(c->flags, frac, res + sizeof(Counts), s1, g, c->stream));
+        HIP_TRY(c, setup_clean(c->flags, c->rowclean, res + sizeof(Counts) + nblk, g, c->stream));
+        HIP_TRY(c, hipMemcpyAsync(got.data(), res, hold, hipMemcpyDeviceToHost, c->stream));
         HIP_TRY(c, hipStreamSynchronize(c->stream));
-        if (c->prec != LBM_FP64) {
-            // Dense mode: one per-node pass over every node instead of the copies, the packed pass
-            // and the fix-up of the list, chosen
-            //  * when the fix list holds more than a quarter of the fluid nodes (a solid fraction
-            //    over a noisy field: half of them on the 192x96x96 adjoint workload, where the
-            //    list path took 67 + 100 us per step and the dense pass 67 us), or
-            //  * when a population buffer is at most 16 MB: such steps are launch-bound, and one
-            //    launch fewer per step counts (D2Q9 512x128 with the drag every step: 6.7 / 6.4 us
-            //    per step in FP32 / FP16 against 8.7 / 8.8; on D3Q27 512x128x128 the dense pass
-            //    is as fast in FP32 but 1.5 times slower in FP16, so large domains keep the list).
-            // LBM_DENSE=1 / 0 forces the choice.
-            const size_t pop_bytes = (size_t)(c->prec == LBM_FP32 ? 4 : 2) * Q * g.plane;
-            const bool small = pop_bytes <= ((size_t)16 << 20);
-            const char *dense_env = std::getenv("LBM_DENSE");
-            c->dense = dense_env ? dense_env[0] == '1' : (!all_slow && ((size_t)counts[2] * 4 > c->N - counts[0] || small));
-            per_block = c->dense;
-        }
-        if (per_block) {
-            forced_blk.resize((size_t)s1.gx * g.ny * g.nz);
-            HIP_TRY(c, blk.alloc(forced_blk.size()));
-            HIP_TRY(c, setup_forced(c->flags, (const double *)frac.p, (uint8_t *)blk.p, s1, g, c->stream));
-            HIP_TRY(c, hipMemcpyAsync(forced_blk.data(), blk.p, forced_blk.size(), hipMemcpyDeviceToHost, c->stream));
-            HIP_TRY(c, hipStreamSynchronize(c->stream));
-        }
     }
-    c->solid_nodes = (int)counts[0];
-    c->near_nodes = (int)counts[1];
-    // rows whose nodes are all fluid with no solid neighbour (the adjoint's straight-line rows;
-    // LBM_ADJ_GENERAL_PATH=1 sends every row through the general path, for tests)
-    std::vector<uint8_t> clean((size_t)g.ny * g.nz);
-    HIP_TRY(c, hipMalloc(&c->rowclean, clean.size()));
-    HIP_TRY(c, setup_clean(c->flags, c->rowclean, g, c->stream));
-    HIP_TRY(c, hipMemcpyAsync(clean.data(), c->rowclean, clean.size(), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(c, hipStreamSynchronize(c->stream));
+    std::memcpy(&counts, got.data(), sizeof(counts));
+    const uint8_t *const forced_blk = got.data() + sizeof(Counts);   // per block of shape s1: holds a forced node
+    uint8_t *const clean = got.data() + sizeof(Counts) + nblk;       // per row: all nodes fluid with no solid neighbour
+    c->solid_nodes = (int)counts.solid;
+    c->near_nodes = (int)counts.near;
+    // Dense mode: one per-node pass over every node instead of the copies, the packed pass
+    // and the fix-up of the list, chosen
+    //  * when the fix list holds more than a quarter of the fluid nodes (a solid fraction
+    //    over a noisy field: half of them on the 192x96x96 adjoint workload, where the
+    //    list path took 67 + 100 us per step and the dense pass 67 us), or
+    //  * when a population buffer is at most 16 MB: such steps are launch-bound, and one
+    //    launch fewer per step counts (D2Q9 512x128 with the drag every step: 6.7 / 6.4 us
+    //    per step in FP32 / FP16 against 8.7 / 8.8; on D3Q27 512x128x128 the dense pass
+    //    is as fast in FP32 but 1.5 times slower in FP16, so large domains keep the list).
+    // LBM_DENSE=1 / 0 forces the choice.
+    if (c->prec != LBM_FP64) {
+        const size_t pop_bytes = (size_t)(c->prec == LBM_FP32 ? 4 : 2) * Q * g.plane;
+        const bool small = pop_bytes <= ((size_t)16 << 20);
+        const char *dense_env = std::getenv("LBM_DENSE");
+        c->dense = dense_env ? dense_env[0] == '1' : (!all_slow && ((size_t)counts.fix * 4 > c->N - counts.solid || small));
+    }
+    const bool per_block = c->prec == LBM_FP64 || c->dense;
     // the lists below are per node; a dense or FP64 step needs none
     std::vector<uint8_t> flags;
     std::vector<uint32_t> near_list;   // D3Q27: the nodes next to the mask
@@ -499,7 +493,7 @@ static int init_plain(lbm_ctx *c) {
     std::vector<int> slot;
     c->nslots = 0;
     if (per_block) {
-        slot.resize(forced_blk.size());
+        slot.resize(nblk);
         for (size_t b = 0; b < slot.size(); b++) slot[b] = forced_blk[b] ? c->nslots++ : -1;
     }
     // FP32/16-bit: per fluid node (row-major padded indices), either
@@ -671,9 +665,11 @@ static int init_plain(lbm_ctx *c) {
                              per_block && !sf ? slot : std::vector<int>(), s1, c->stream));
     }
     {
+        // (the adjoint's straight-line rows; LBM_ADJ_GENERAL_PATH=1 sends every row through the general
+        // path, for tests)
         if (std::getenv("LBM_ADJ_GENERAL_PATH")) {
-            std::fill(clean.begin(), clean.end(), (uint8_t)0);
-            HIP_TRY(c, hipMemcpy(c->rowclean, clean.data(), clean.size(), hipMemcpyHostToDevice));
+            std::fill(clean, clean + nrow, (uint8_t)0);
+            HIP_TRY(c, hipMemcpy(c->rowclean, clean, nrow, hipMemcpyHostToDevice));
         }
         c->adj_all_fast = true;
         for (int z = 0; z < g.nz; z++)

@@ -7,9 +7,10 @@
 
 namespace lbm {
 
-// solid or fluid; the padding of a row is solid
+// solid or fluid; the padding of a row is solid.  Clears the counts of the next launch.
 __global__ void __launch_bounds__(256) k_setup_solid(uint8_t *__restrict__ flags, const uint8_t *__restrict__ mask, SetupBody b, Geo g,
-                                                     int D) {
+                                                     int D, unsigned *__restrict__ counts) {
+    if (blockIdx.x + blockIdx.y + blockIdx.z == 0 && threadIdx.x < 3) counts[threadIdx.x] = 0u;
     const int x = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y, z = blockIdx.z;
     if (x >= g.nxp) return;
     const size_t row = (size_t)y + (size_t)g.ny * z;
@@ -78,12 +79,13 @@ __global__ void __launch_bounds__(256) k_setup_forced(const uint8_t *__restrict_
 }
 
 // per row: 1 when every node is fluid with no solid neighbour
-__global__ void __launch_bounds__(256) k_setup_clean(const uint8_t *__restrict__ flags, uint8_t *__restrict__ clean, Geo g) {
+__global__ void __launch_bounds__(256) k_setup_clean(const uint8_t *__restrict__ flags, uint8_t *__restrict__ clean,
+                                                     uint8_t *__restrict__ copy, Geo g) {
     const size_t row = (size_t)blockIdx.x + (size_t)g.ny * blockIdx.y;
     bool bad = false;
     for (int x = threadIdx.x; x < g.nx; x += 256) bad = bad || flags[(size_t)x + (size_t)g.nxp * row] != FL_FLUID;
     const int any = __syncthreads_or(bad);
-    if (threadIdx.x == 0) clean[row] = any ? 0 : 1;
+    if (threadIdx.x == 0) clean[row] = copy[row] = any ? 0 : 1;
 }
 
 __global__ void __launch_bounds__(256) k_setup_links9(const uint8_t *__restrict__ flags, uint16_t *__restrict__ lk, Geo g) {
@@ -124,9 +126,7 @@ static dim3 row_blocks(const Geo &g) { return dim3((unsigned)((g.nxp + 255) / 25
 
 hipError_t setup_flags(int Q, uint8_t *flags, const uint8_t *mask, const double *sfrac, const SetupBody &b, const SetupFix &fix,
                        const Geo &g, unsigned *counts, hipStream_t s) {
-    hipError_t e = hipMemsetAsync(counts, 0, 3 * sizeof(unsigned), s);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_setup_solid, row_blocks(g), dim3(256), 0, s, flags, mask, b, g, Q == 9 ? 2 : 3);
+    hipLaunchKernelGGL(k_setup_solid, row_blocks(g), dim3(256), 0, s, flags, mask, b, g, Q == 9 ? 2 : 3, counts);
     if (Q == 9) hipLaunchKernelGGL(k_setup_near<9>, row_blocks(g), dim3(256), 0, s, flags, sfrac, g, fix, counts);
     else hipLaunchKernelGGL(k_setup_near<27>, row_blocks(g), dim3(256), 0, s, flags, sfrac, g, fix, counts);
     return hipGetLastError();
@@ -138,8 +138,8 @@ hipError_t setup_forced(const uint8_t *flags, const double *sfrac, uint8_t *out,
     return hipGetLastError();
 }
 
-hipError_t setup_clean(const uint8_t *flags, uint8_t *clean, const Geo &g, hipStream_t s) {
-    hipLaunchKernelGGL(k_setup_clean, dim3((unsigned)g.ny, (unsigned)g.nz), dim3(256), 0, s, flags, clean, g);
+hipError_t setup_clean(const uint8_t *flags, uint8_t *clean, uint8_t *copy, const Geo &g, hipStream_t s) {
+    hipLaunchKernelGGL(k_setup_clean, dim3((unsigned)g.ny, (unsigned)g.nz), dim3(256), 0, s, flags, clean, copy, g);
     return hipGetLastError();
 }
 
