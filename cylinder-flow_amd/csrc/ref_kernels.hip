@@ -236,8 +236,10 @@ __global__ void __launch_bounds__(256) k_ref_usrbc(RefGeo r, double *__restrict_
 }
 
 // usrbc over a list of the nodes it can change (interior solid nodes with a fluid neighbour,
-// node indices built once from usr): the same per-node work as k_ref_usrbc without sweeping
-// the interior
+// node indices built once from usr): the copies of k_ref_usrbc without sweeping the interior, one lane per
+// node and direction (blockIdx.y).  No copy reads a slot that another writes (the host's check), so they
+// need no order; a lane per node ran its 26 copies one after another, each waiting for the last
+// (512x128x128, a sphere of radius 8: 21.2 us against 4.4 of the 722 of a step).
 template <int Q>
 __global__ void __launch_bounds__(256) k_ref_usrbc_list(RefGeo r, double *__restrict__ f, const uint8_t *__restrict__ usr,
                                                         const uint32_t *__restrict__ list, int nlist) {
@@ -247,8 +249,9 @@ __global__ void __launch_bounds__(256) k_ref_usrbc_list(RefGeo r, double *__rest
     const uint32_t node = list[t], row = node / (uint32_t)r.px;
     const int i = (int)(node - row * (uint32_t)r.px), j = (int)(row % (uint32_t)r.ly), k = (int)(row / (uint32_t)r.ly);
     const long n = (long)node;
-    static_for<0, Q>([&](auto I) {
+    static_for<1, Q>([&](auto I) {
         constexpr int ii = I;
+        if ((int)blockIdx.y + 1 != ii) return;
         const long nb = n + L::ex(ii) + (long)r.px * (L::ey(ii) + (long)r.ly * L::ez(ii));
         if (usr[nb] == 1)
             f[RIDX(r, ii, i, j, k)] = f[RIDX(r, L::opp(ii), i + 2 * L::ex(ii), j + 2 * L::ey(ii), k + 2 * L::ez(ii))];
@@ -591,7 +594,7 @@ hipError_t ref_fills(const RefGeo &r, double *f, double *ft, hipStream_t s) {
 hipError_t ref_usrbc(const RefGeo &r, double *f, const uint8_t *usr, const uint32_t *list, int nlist, hipStream_t s) {
     if (list) {   // the listed nodes only (none: nothing to do)
         if (nlist == 0) return hipSuccess;
-        const dim3 grid((unsigned)((nlist + 255) / 256));
+        const dim3 grid((unsigned)((nlist + 255) / 256), (unsigned)(r.Q - 1));
         if (r.Q == 9) hipLaunchKernelGGL(k_ref_usrbc_list<9>, grid, dim3(256), 0, s, r, f, usr, list, nlist);
         else hipLaunchKernelGGL(k_ref_usrbc_list<27>, grid, dim3(256), 0, s, r, f, usr, list, nlist);
         return hipGetLastError();
