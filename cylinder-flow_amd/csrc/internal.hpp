@@ -162,12 +162,12 @@ hipError_t pair_plan(PairPlan &p, int prec, const Geo &g, const uint8_t *flags, 
 // fills p.bw, p.tflag and p.linklk (pair_words.hip)
 hipError_t pair_words(const PairPlan &p, const PairOps &ops, const uint8_t *flags, const Geo &g, hipStream_t s);
 void pair_free(PairPlan &p);
-// several D2Q9 steps per launch (small_kernel.hpp): tb_depth() steps at most, T x T tiles
-// (tb_tile), tb_tiles(g, T, K) blocks with tb_lds_bytes(prec, T) of LDS each
-int tb_depth();
+// several D2Q9 steps per launch (small_kernel.hpp): K steps at most, T x T tiles
+// (tb_choose), tb_tiles(g, T, K) blocks with tb_lds_bytes(prec, T) of LDS each
 size_t tb_lds_bytes(int prec, int T);
 int tb_tiles(const Geo &g, int T, int K, int *tiles_x);
-int tb_tile(const Geo &g, int K, int cus);
+// steps per launch and tile side of a domain with the force every fi steps (0: never)
+void tb_choose(const Geo &g, int prec, int fi, int cus, int &K, int &T);
 // before the first launch: the LDS limit of the kernels for side T (sfrac: null or not) on this device
 hipError_t tb_prepare(int prec, int T, const void *sfrac, const FusedArgs &a);
 // tb_steps: `steps` (<= K) steps in one launch; the partials of its force records go to record

@@ -397,16 +397,6 @@ FusedArgs ctx_fused_args(const lbm_ctx *c) {
     return a;
 }
 
-struct DevTmp {   // device memory of a scope
-    void *p = nullptr;
-    DevTmp() = default;
-    DevTmp(const DevTmp &) = delete;
-    ~DevTmp() {
-        if (p) (void)hipFree(p);
-    }
-    hipError_t alloc(size_t n) { return hipMalloc(&p, n); }
-};
-
 static int init_plain(lbm_ctx *c) {
     const Geo &g = c->geo;
     const int Q = c->Q;
@@ -424,18 +414,19 @@ static int init_plain(lbm_ctx *c) {
     // (the reference's "usr", 3D MPI+KOKKOS+MPIIO/lbm.cpp:238) or the user mask
     HIP_TRY(c, hipMalloc(&c->flags, g.plane));
     const Shape s1 = c->prec == LBM_FP64 ? fp64_shape(g, Q) : lane_shape(g, 1);
-    // one scratch buffer; what the host reads of it comes back in one copy
+    // what the host reads of it comes back in one copy
     struct Counts {
         unsigned solid, near, fix;   // nodes of each kind, nodes of the fix list
     } counts;
     const size_t nblk = (size_t)s1.gx * g.ny * g.nz, nrow = (size_t)g.ny * g.nz, hold = sizeof(Counts) + nblk + nrow;
     std::vector<uint8_t> got(hold);
     {
-        const size_t fracb = sf ? sizeof(double) * c->N : 0, maskb = c->cfg.body == LBM_BODY_MASK ? c->N : 0;
-        DevTmp tmp;   // solid fraction, counts, force blocks, clean rows, mask
-        HIP_TRY(c, tmp.alloc(fracb + hold + maskb));
-        double *const frac = sf ? (double *)tmp.p : nullptr;
-        uint8_t *const res = (uint8_t *)tmp.p + fracb, *const mask = maskb ? res + hold : nullptr;
+        // the moment planes (32 bytes per padded node, 64 of them a row at least), which nothing uses yet,
+        // hold the scratch: solid fraction, counts, force blocks, clean rows, mask
+        HIP_TRY(c, hipMalloc(&c->macros, sizeof(double) * 4 * g.plane));
+        const size_t fracb = sizeof(double) * c->N;
+        double *const frac = sf ? c->macros : nullptr;
+        uint8_t *const res = (uint8_t *)c->macros + fracb, *const mask = c->cfg.body == LBM_BODY_MASK ? res + hold : nullptr;
         if (mask) HIP_TRY(c, hipMemcpyAsync(mask, c->solid.data(), c->N, hipMemcpyHostToDevice, c->stream));
         if (sf) {
             HIP_TRY(c, hipMemcpyAsync(frac, c->sfrac.data(), sizeof(double) * c->N, hipMemcpyHostToDevice, c->stream));
@@ -594,16 +585,17 @@ static int init_plain(lbm_ctx *c) {
     }
     // D2Q9 on a small domain, where a step costs about a dependent launch: several steps per launch
     // (temporal blocking, small_kernel.hpp), for walls, inlet, outlet, a mask and a solid fraction,
-    // up to 420 000 nodes (padded).  On larger ones, and where an axis is periodic, STRIP_K steps per
-    // pass over memory (strip_kernel.hpp), from 360 000 nodes on, in 16-bit storage from 3 million.
-    // us per step with drag every 10 steps, one launch per step / tiles / strips:
-    //               FP64                 FP32                 FP16
-    //   600x150     5.76 / 3.74 / 8.3    4.68 / 1.86 / 5.4    4.47 / 1.95 / 5.8
-    //   1000x250    9.80 / 7.96 / 11.2   6.38 / 4.60 / 6.2    5.64 / 5.06 / 6.6
-    //   1200x300    12.0 / 10.6 / 11.5   7.84 / 5.67 / 6.3    6.82 / 6.41 / 6.7
-    //   1400x350    15.8 / 14.7 / 12.9   9.26 / 7.70 / 7.5    8.28 / 8.65 / 8.5
-    //   2000x500    27.3 / 29.3 / 19.7   15.1 / 15.2 / 10.1   9.99 / 15.9 / 12.0
-    //   2048x2048   100 / 110 / 55.4     50.4 / 56.6 / 24.5   27.0 / 59.8 / 25.1
+    // up to 420 000 nodes (padded), in FP32 330 000.  On larger ones, and where an axis is periodic,
+    // STRIP_K steps per pass over memory (strip_kernel.hpp), from 360 000 nodes on, in FP32 from 330 000 and
+    // in 16-bit storage from 3 million.  us per step with drag every 10 steps, one launch per step / tiles / strips
+    // (in brackets tiles / strips with the drag every step, where the order changes):
+    //               FP64                 FP32                            FP16
+    //   600x150     5.76 / 2.54 / 7.4    4.68 / 1.65 / 5.2               4.47 / 1.73 / 5.5
+    //   1000x250    9.80 / 6.22 / 11.0   6.38 / 3.67 / 6.1               5.64 / 3.99 / 6.5
+    //   1200x300    12.0 / 9.32 / 11.2   7.84 / 6.26 / 6.2 (8.5 / 6.8)   6.82 / 6.48 / 6.6 (8.5 / 7.2)
+    //   1400x350    15.8 / 12.7 / 12.3   9.26 / 5.92 / 7.3 (8.0 / 8.0)   8.28 / 5.48 / 8.3 (7.6 / 9.0)
+    //   2000x500    27.3 / 21.6 / 16.4   15.1 / 18.7 / 9.1               9.99 / 16.7 / 11.2
+    //   2048x2048   100 / - / 55.4       50.4 / - / 24.5                 27.0 / - / 25.1
     // LBM_TEMPORAL_BLOCKING=0 keeps one step per launch, 1 / 2 take the tiles / the strips
     // regardless of the size.
     {
@@ -616,8 +608,8 @@ static int init_plain(lbm_ctx *c) {
                 eligible = eligible && std::getenv(k) == nullptr;
             eligible = eligible && (c->prec == LBM_FP32 || c->cfg.store_uref == 0.0);
         }
-        const bool small = g.plane <= 420000, tiles_ok = eligible && !g.xper && !g.yper;
-        const bool large = g.plane >= (c->prec == LBM_FP64 || c->prec == LBM_FP32 ? 360000u : 3000000u);
+        const bool small = g.plane <= (c->prec == LBM_FP32 ? 330000u : 420000u), tiles_ok = eligible && !g.xper && !g.yper;
+        const bool large = g.plane >= (c->prec == LBM_FP64 ? 360000u : c->prec == LBM_FP32 ? 330000u : 3000000u);
         const size_t esz9 = c->prec == LBM_FP64 ? 8 : c->prec == LBM_FP32 ? 4 : 2;
         int dev = 0, lds_max = 0;
         if (eligible && (hipGetDevice(&dev) != hipSuccess ||
@@ -626,8 +618,9 @@ static int init_plain(lbm_ctx *c) {
             eligible = false;
         int nparts = 0, slots = 0;
         if (eligible && tiles_ok && (tbe ? tbe[0] == '1' : small)) {
-            const int K = tb_depth(), T = tb_tile(g, K, c->cus);
-            if ((size_t)lds_max >= tb_lds_bytes(c->prec, T) + 4096 + 512 &&
+            int K = 0, T = 0;
+            tb_choose(g, c->prec, c->cfg.force_interval, c->cus, K, T);
+            if (K > 0 && (size_t)lds_max >= tb_lds_bytes(c->prec, T) + 4096 + 512 &&
                 tb_prepare(c->prec, T, sf ? c : nullptr, ctx_fused_args(c)) == hipSuccess) {
                 c->tb_k = K;
                 c->tb_t = T;
@@ -655,7 +648,6 @@ static int init_plain(lbm_ctx *c) {
     HIP_TRY(c, hipMalloc(&c->A, esz * Q * g.plane));
     HIP_TRY(c, hipMalloc(&c->B, esz * Q * g.plane));
     HIP_TRY(c, hipMalloc(&c->duin, sizeof(double) * c->uin.size()));
-    HIP_TRY(c, hipMalloc(&c->macros, sizeof(double) * 4 * g.plane));
     HIP_TRY(c, hipMalloc(&c->block_slot, sizeof(int) * std::max<size_t>(slot.size(), 1)));
     HIP_TRY(c, hipMalloc(&c->partials, force_bytes(c->nslots)));
     // D3Q27: two steps per pass over memory where the two-step kernel applies (pair.cpp); its force

@@ -4,7 +4,7 @@
 // so a step costs what a dependent launch costs (~3.4 us on one MI355X; a captured graph of
 // launches costs the same).  Temporal blocking removes all but one launch per K steps: block b
 // owns a W x W core of nodes and loads its core plus a halo of K nodes on each side (T x T
-// nodes, T = 24..32, the side with the least rounds of the CUs times T^2) into the LDS,
+// nodes, T = 24..32, K and T chosen for the domain by tb_choose) into the LDS,
 // coalesced; each of the K steps pulls from the LDS (boundary rules applied by the values the
 // live nodes write, setup_links9) and collides in registers (one thread per node), and the live
 // nodes write their populations back to the LDS.  A halo node's result is exact as long as every node it pulled from was, so the exact
@@ -21,7 +21,7 @@
 
 namespace lbm {
 
-constexpr int TB_KMAX = 10;   // steps per launch at most (tb_depth)
+constexpr int TB_KMAX = 10;   // steps per launch at most (tb_choose)
 
 // LDS row length (doubles) of a T x T tile: the odd one of T + 1, T + 2
 __host__ __device__ constexpr int tb_row(int T) { return T % 2 == 0 ? T + 1 : T + 2; }
@@ -256,7 +256,8 @@ __global__ void __launch_bounds__(1024)
                     });
             }
             __syncthreads();
-            if (keep != nullptr) store_core(buf, keep + keep_stride * (size_t)(s - 1));
+            if constexpr (!ANY_FORCE)   // (states are kept without force records)
+                if (keep != nullptr) store_core(buf, keep + keep_stride * (size_t)(s - 1));
         }
         double fx = 0.0, fy = 0.0;
         if (dist <= rs && live) {

@@ -30,17 +30,6 @@ __global__ void __launch_bounds__(256) k_tb_force(const double *__restrict__ par
     }
 }
 
-// steps per launch: 7 (LBM_TB_DEPTH overrides, 1-10); FP64: with the 14 x 14 core of a 400 x 100
-// domain's 28 x 28 tiles, 7 steps per launch measured fastest (2.54 us per step against 2.61 at
-// 5 steps on 24 x 24 tiles and 2.60 at 8 on 30 x 30)
-int tb_depth() {
-    if (const char *e = std::getenv("LBM_TB_DEPTH")) {
-        const int k = std::atoi(e);
-        if (k >= 1 && k <= TB_KMAX) return k;
-    }
-    return 7;
-}
-
 size_t tb_lds_bytes(int prec, int T) { return tb_lds_size(T, prec == LBM_FP64 ? 8 : prec == LBM_FP32 ? 4 : 2); }
 
 hipError_t tb_launch_f64(const TbLaunch &l, const FusedArgs &a, hipStream_t s);
@@ -54,29 +43,53 @@ int tb_tiles(const Geo &g, int T, int K, int *tiles_x) {
     return *tiles_x * ((g.ny + W - 1) / W);
 }
 
-// the tile sides instantiated, and the tile side for a domain (leaving a core of at least 2 x 2
-// nodes); LBM_TB_TILE overrides with any instantiated side that leaves a 2 x 2 core
+// Steps per launch and tile side of a domain: the least microseconds per step by a model of a launch of K
+// steps over T x T tiles, in rounds of one tile per CU (FP64, whose tile fills the LDS) or two:
+//   t0 + rounds of the CUs * a K + tiles per CU * b * wave-steps of the busiest SIMD (+ c T^2 per round, FP64),
+// a and b larger by a1, b1 in a step that records the force.  The constants are a least-squares fit to 126
+// launches per format from 48x32 to 1000x250, 4 to 10 steps, the force every step and every 10 (FP64: 2 % rms,
+// FP32 and 16 bits: 9 %).  More steps save launches, until the halo makes the tiles too many for the CUs: us
+// per step with the force every 10 steps, always 7 steps per launch / this choice:
+//              FP64           FP32           FP16
+//   48x32      1.78 / 1.51    1.28 / 1.06    1.41 / 1.13
+//   400x100    2.03 / 1.93    1.38 / 1.31    1.51 / 1.40
+//   512x128    2.38 / 2.25    1.55 / 1.48    1.68 / 1.58
+//   600x150    3.78 / 2.54    1.89 / 1.65    2.03 / 1.73
+//   800x200    5.68 / 4.02    2.80 / 2.66    2.99 / 2.73
+//   1000x250   8.05 / 6.22    4.97 / 3.67    5.53 / 3.99
+// (with the force every step 10.7 / 7.51, 8.20 / 4.70 and 8.35 / 4.67 on the last; a few percent of each is
+// the kept states' test, which launches with force records no longer hold).  t0 lies 0.3 (FP64) below and 0.8
+// above the fit's, where the least measured launches of 400x100 and 512x128 are taken.
+// LBM_TB_DEPTH (1-10) fixes the steps, LBM_TB_TILE the side (one that is instantiated and leaves a 2 x 2 core).
 static const int kTbSides[] = {24, 25, 26, 27, 28, 29, 30, 31, 32};
 
-int tb_tile(const Geo &g, int K, int cus) {
-    if (const char *e = std::getenv("LBM_TB_TILE")) {
-        const int t = std::atoi(e);
-        for (int T : kTbSides)
-            if (t == T && t - 2 * K >= 2) return t;
-    }
-    // the side with the least (rounds of the CUs) x (positions per tile); measured best on
-    // 400 x 100 (27), 600 x 150 (28), 800 x 200 (29) and 1000 x 250 (30) at 7 steps per launch
-    int best = 32, tx = 0;
-    long best_cost = -1;
-    for (int T : kTbSides) {
-        if (T - 2 * K < 2) continue;
-        const long rounds = (tb_tiles(g, T, K, &tx) + cus - 1) / cus, cost = rounds * T * T;
-        if (best_cost < 0 || cost < best_cost) {
-            best = T;
-            best_cost = cost;
+void tb_choose(const Geo &g, int prec, int fi, int cus, int &K, int &T) {
+    const bool f64 = prec == LBM_FP64;
+    const double phi = fi > 0 ? 1.0 / fi : 0.0;
+    const double t0 = f64 ? 2.2 : 3.2, a = f64 ? 0.606 + 0.288 * phi : 0.494 + 0.08 * phi,
+                 b = f64 ? 0.287 + 0.185 * phi : 0.304 + 0.32 * phi, c = f64 ? 0.0042 : 0.0;
+    int only_k = 0, only_t = 0;
+    if (const char *e = std::getenv("LBM_TB_DEPTH")) only_k = std::atoi(e);
+    if (only_k < 1 || only_k > TB_KMAX) only_k = 0;
+    if (const char *e = std::getenv("LBM_TB_TILE"))
+        for (int side : kTbSides)
+            if (std::atoi(e) == side && (only_k ? side - 2 * only_k : side - 4) >= 2) only_t = side;
+    double best = -1.0;
+    K = T = 0;
+    for (int k = only_k ? only_k : 2; k <= (only_k ? only_k : TB_KMAX); k++)
+        for (int side : kTbSides) {
+            const int W = side - 2 * k;
+            if (W < 2 || (only_t && side != only_t)) continue;
+            int tx = 0, waves = 0;
+            const int n = tb_tiles(g, side, k, &tx), per_cu = (n + cus - 1) / cus, at_once = f64 ? 1 : 2;
+            for (int m = 0; m < k; m++) waves += ((W + 2 * m) * (W + 2 * m) + 255) / 256;
+            const double t = (t0 + (per_cu + at_once - 1) / at_once * a * k + per_cu * (b * waves + c * side * side)) / k;
+            if (best < 0.0 || t < best) {
+                best = t;
+                K = k;
+                T = side;
+            }
         }
-    }
-    return best;
 }
 
 // record slots of the partials buffer: the force records of several launches are summed by one
@@ -114,7 +127,7 @@ hipError_t tb_steps(int prec, const void *A, void *B, const uint8_t *flags, cons
     const int nforce = fi > 0 ? (int)((step0 + steps) / fi - step0 / fi) : 0;
     *nrec = nforce;
     if (pend < 0 || pend + nforce > tb_records(K)) return hipErrorInvalidValue;
-    if (T - 2 * K < 1 || K > TB_KMAX || steps < 1 || steps > K) return hipErrorInvalidValue;
+    if (T - 2 * K < 1 || K > TB_KMAX || steps < 1 || steps > K || (keep && nforce > 0)) return hipErrorInvalidValue;
     return tb_launch(prec, TbLaunch{A, B, flags, lk, sfrac, uin, partials, keep, keep_stride, T, K, steps, fi, tiles_x, ntiles, pend,
                                     step0, nforce > 0, false}, a, s);
 }
