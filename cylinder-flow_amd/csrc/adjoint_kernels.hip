@@ -40,8 +40,8 @@ static AdjTab adj_tab(const Geo &g) {
     return t;
 }
 
-// Rows whose nodes are all fluid and have no solid neighbour ("clean", flagged per row on the
-// host) and that are not on a periodic y/z edge take a straight-line path: every source and
+// Rows whose nodes are all fluid and have no solid neighbour ("clean", flagged per row at
+// initialisation) and that are not on a periodic y/z edge take a straight-line path: every source and
 // destination row of a direction is a scalar of the block (at a y/z wall, the node's own row and
 // the opposite direction: half-way bounce-back), and the x edges (inlet, outlet, periodic x) are
 // handled with in-row clamped indices and selects, so every load of the path is issued

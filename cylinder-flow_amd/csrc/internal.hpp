@@ -155,9 +155,9 @@ struct PairOps {   // a storage format's column, LDS bytes and launchers
 };
 PairOps pair_ops(int prec);
 // the plan of a domain; p.on stays false where the two-step kernel does not apply (pair.cpp).
-// flags: on the device, complete on stream s; near_nodes: the nodes next to the mask, in node order;
+// flags: on the device, complete on stream s; packed: the one-step path is k_fast_v alone; near_nodes: the nodes next to the mask, in node order;
 // block_slot: the one-step path's slot per block of shape `blk` (empty: its slots are per node)
-hipError_t pair_plan(PairPlan &p, int prec, const Geo &g, const uint8_t *flags, bool same_offsets,
+hipError_t pair_plan(PairPlan &p, int prec, const Geo &g, const uint8_t *flags, bool same_offsets, bool packed,
                      const std::vector<uint32_t> &near_nodes, const std::vector<int> &block_slot, Shape blk, hipStream_t s);
 // fills p.bw, p.tflag and p.linklk (pair_words.hip)
 hipError_t pair_words(const PairPlan &p, const PairOps &ops, const uint8_t *flags, const Geo &g, hipStream_t s);

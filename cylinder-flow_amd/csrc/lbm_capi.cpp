@@ -653,7 +653,7 @@ static int init_plain(lbm_ctx *c) {
     // D3Q27: two steps per pass over memory where the two-step kernel applies (pair.cpp); its force
     // slots are those of the one-step path
     if (Q == 27) {
-        HIP_TRY(c, pair_plan(c->pair, c->prec, g, c->flags, same_offsets, sf ? std::vector<uint32_t>() : near_list,
+        HIP_TRY(c, pair_plan(c->pair, c->prec, g, c->flags, same_offsets, !per_block && c->nfix == 0, sf ? std::vector<uint32_t>() : near_list,
                              per_block && !sf ? slot : std::vector<int>(), s1, c->stream));
     }
     {

@@ -30,11 +30,26 @@ static hipError_t upload(T *&dst, const std::vector<T> &src) {
     return e;
 }
 
-hipError_t pair_plan(PairPlan &p, int prec, const Geo &g, const uint8_t *flags, bool same_offsets,
+// Whether two steps per pass take less time than two one-step launches: a pass takes 9 us (FP64), 5 (FP32) or
+// 4.25 (16 bits) per plane of work and round, a one-step launch a few us and then its share per 1000
+// padded nodes; in 16 bits that holds for the packed kernel alone (dense mode and a fix-up list are
+// slower at every size measured).  Two columns of few planes each redo most of their first step: us per
+// step, one step per launch / two steps per pass, on 40 domains from 24x16x16 to 320x140x140 (the constants
+// follow them): FP64 24x16x16 7.2 / 12.1, 40x123x30 18.8 / 21.9, 96x48x48 22.4 / 21.6, 125x67x45 33.5 / 30.5,
+// 320x140x140 548 / 377; FP32 61x23x22 7.0 / 7.9, 33x53x28 8.3 / 8.4, 125x67x45 19.2 / 14.1; FP16 packed
+// 222x17x124 15.8 / 18.4, 320x140x140 120 / 128 (two rounds), 192x96x96 38.3 / 35.1.
+static bool pair_pays(int prec, const Geo &g, long cost, bool packed) {
+    const double k = 1e-3 * (double)g.plane;
+    if (prec == LBM_FP64) return 9.0 * cost / 2 < 5.5 + 0.068 * k;
+    if (prec == LBM_FP32) return 5.0 * cost / 2 < 6.2 + 0.031 * k;
+    return !packed || 4.25 * cost / 2 < 4.0 + 0.0195 * k;
+}
+
+hipError_t pair_plan(PairPlan &p, int prec, const Geo &g, const uint8_t *flags, bool same_offsets, bool packed,
                      const std::vector<uint32_t> &near_nodes, const std::vector<int> &block_slot, Shape blk, hipStream_t s) {
     pair_free(p);
-    // LBM_TWO_STEPS=0 keeps one step per launch; so does any switch that selects among the one-step
-    // kernels.  Opposite directions must share their storage offset (a bounced value is taken as
+    // LBM_TWO_STEPS=0 keeps one step per launch, 1 takes two per pass whether or not that pays; any switch
+    // that selects among the one-step kernels keeps one.  Opposite directions must share their storage offset (a bounced value is taken as
     // stored), the rows must be interleaved, and the buffers' byte offsets must fit 32 bits: the
     // three planes a pull spans, with periodic z the whole state.
     const char *env = std::getenv("LBM_TWO_STEPS");
@@ -68,6 +83,7 @@ hipError_t pair_plan(PairPlan &p, int prec, const Geo &g, const uint8_t *flags, 
             p.chunks = m;
         }
     }
+    if (!(env && env[0] == '1') && !pair_pays(prec, g, best, packed)) return hipSuccess;
     // bounce words, column bits and the links of the listed nodes, on the device
     const size_t words = (size_t)((g.nz + 31) / 32) * (size_t)tiles;
     if (near_nodes.size() > (size_t)INT32_MAX) return hipSuccess;

@@ -22,8 +22,8 @@
 // more than the plain pull; elsewhere the pull has no rule but the x edges: the inlet's unknowns are overwritten by the inlet rule, the outlet's source is
 // clamped and periodic axes wrap, all three in the lane's offsets.
 //
-// 512x256x256 cylinder, us per step, one step per launch / two: FP64 2525 / 1825, FP32 1197 / 871,
-// FP16 630 / 569.  FP32 is bound by HBM (5.4 TB/s of L2 misses with every block in step; the rim reads
+// 512x256x256 cylinder, us per step, one step per launch / two: FP64 2525 / 1735, FP32 1197 / 875,
+// FP16 630 / 572.  FP32 is bound by HBM (5.4 TB/s of L2 misses with every block in step; the rim reads
 // 1.13 times the state), FP16 by instruction issue (68 % VALU busy at 309 instructions per node and
 // step), FP64 by both.
 //

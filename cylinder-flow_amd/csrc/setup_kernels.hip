@@ -1,7 +1,9 @@
 // setup_kernels.hip -- initialisation of the plain mode's node arrays on the device: node flags from the
 // body formula or the mask, the padded solid fraction, and the per-row and per-block predicates that the
 // host's lists are built from.  (3D MPI+KOKKOS+MPIIO/lbm.cpp:238 for the "usr" formula.)  On the host the
-// same classification took 26 neighbour tests per node: 80 ms at 192x96x96, 1.3 s at 512x256x256.
+// same classification, up to 26 neighbour tests per node, took 78 of the 80 ms of an initialisation at
+// 192x96x96 (now 1.9 ms in all) and 0.5 of 0.77 ms at 400x100 (0.20).  One lane per node in blocks of 256
+// along a row: bound by the flags' bytes and by launches, so nothing is staged.
 #include "internal.hpp"
 #include "lattice.hpp"
 

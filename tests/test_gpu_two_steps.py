@@ -50,7 +50,7 @@ def test_two_steps_per_pass_equal_one(pkg, monkeypatch, prec, case):
     L = pkg.lbm
     monkeypatch.setenv("LBM_TWO_STEPS", "0")
     a, fa = run(L, L.PRECISIONS[prec], **CASES[case])
-    monkeypatch.delenv("LBM_TWO_STEPS")
+    monkeypatch.setenv("LBM_TWO_STEPS", "1")
     b, fb = run(L, L.PRECISIONS[prec], **CASES[case])
     for x, y in zip(a, b):
         assert np.array_equal(x, y)
