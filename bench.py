@@ -7,16 +7,15 @@ z-spanning cylinder D=40 at (128,128), Re=300, u=0.05, half-way bounce-back on t
 four side walls, Zou-He inlet (regularised), zero-gradient outlet, drag/lift every 10 steps.  Synthetic
 initial state (seeded perturbation); the populations are resident in HBM before timing starts.
 
-A "step" is one fused lattice update of the whole domain: the bounce-back copies into the solid
-slots (k_link_pairs, or k_link_v with the momentum exchange on force steps), k_fast_v (packed
-pull-collide-store over every node) and, when its list is not empty, k_fix_v, back to back on
-the solver's stream.  MLUPS = nodes * steps / seconds over
-exactly --steps steps bracketed by stream synchronisation.  The roofline is that of the
-dominant kernel, k_fast_v: the algorithmic 2*Q*sizeof(storage) bytes per node update times the
-nodes one launch updates, over its average launch duration measured with HIP events recorded
-just before and after each launch on the solver's own stream (a second context with forces
-off).  roofline.step gives the same for the whole step (events around the steps), and
-roofline.traffic the counter-measured HBM bytes per launch (profiles/traffic.json).
+A "step" is one lattice update of the whole domain.  The solver advances two of them per launch of
+k_pair, which reads and writes the state once; a step whose force is recorded second in its pair, and
+the last of an odd count, run alone in k_fast_v (with k_link_force before it on force steps).
+MLUPS = nodes * steps / seconds over exactly --steps steps bracketed by device synchronisation.  The
+roofline is that of the dominant kernel, k_pair: the algorithmic 2*Q*sizeof(storage) bytes per node
+and launch (two updates) times the nodes, over its launch duration (HIP events around an even number of
+steps on the solver's own stream, a second context with forces off: launches of k_pair alone).
+roofline.one_step gives the same for one update per launch (k_fast_v, events just before and after each
+launch), and traffic the counter-measured HBM bytes per launch (profiles/traffic.json).
 """
 from __future__ import annotations
 
@@ -80,21 +79,31 @@ def run_leg(pkg, precision, steps, warmup, force_interval):
     return s, W, wall, info
 
 
-def kernel_roofline(pkg, precision, steps, bytes_per_update, nodes):
-    """Forces off, HIP events on the solver's stream: the average duration of the dominant
-    kernel (k_fast_v, events recorded just before and after each launch) and of the whole step
-    (k_link_pairs + k_fast_v, events around the steps, in a run without the per-kernel events).
-    Returns (kernel seconds, kernel GB/s, step seconds, step GB/s) per launch / step."""
+def kernel_roofline(pkg, precision, steps, bytes_per_update, nodes, kernel, one_step_kernel, limit, traffic):
+    """Forces off, HIP events on the solver's stream: the average duration of a two-step launch of the
+    dominant kernel (events around an even number of steps) and of a one-step launch (events just
+    before and after each; the per-launch events keep one step per launch)."""
     W = pkg.configs.zcylinder3d_512x256x256(precision=precision, force_interval=0)
     s = pkg.Solver(W.cfg).initialize()
-    s.step(5)
-    ms_step = s.step_timed(steps)
-    _, ms_kernel = s.step_kernel_timed(steps)
+    s.step(6)
+    n = steps + steps % 2
+    pair = s.step_timed(n) / n * 2.0 / 1e3
+    _, ms_one = s.step_kernel_timed(steps)
     s.close()
-    per_launch = ms_kernel / steps / 1e3
-    per_step = ms_step / steps / 1e3
+    one = ms_one / steps / 1e3
     algo = bytes_per_update * nodes
-    return per_launch, algo / per_launch / 1e9, per_step, algo / per_step / 1e9
+
+    def entry(name, seconds, updates, tag):
+        gbs = algo / seconds / 1e9
+        return {"bound": "hbm", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                "frac": round(gbs / HBM_PEAK_GBS, 4), "traffic": traffic_from_profiles(tag), "kernel": name,
+                "kernel_ms": round(seconds * 1e3, 5), "bytes_per_update": bytes_per_update / updates,
+                "updates_per_launch": updates}
+
+    out = entry(kernel, pair, 2, f"{traffic}_k_pair")
+    out["limited_by"] = limit
+    out["one_step"] = entry(one_step_kernel, one, 1, f"{traffic}_k_fast_v")
+    return out
 
 
 def traffic_from_profiles(name):
@@ -465,7 +474,6 @@ def main():
     s16.close()
     mlups16 = nodes * K / wall16 / 1e6
     log(f"fp16s {mlups16:.0f} MLUPS, {wall16 / K * 1e3:.4f} ms/step; kernel roofline run")
-    t16, ach16, st16, sach16 = kernel_roofline(pkg, L.FP16S, K, info16.bytes_per_update, nodes)
     out = {
         "metric": METRIC, "value": round(mlups16, 1), "unit": "MLUPS", "n_gpus": 1, "steps": K, "warmup": Wm,
         "ms_per_step": round(wall16 / K * 1e3, 5), "higher_is_better": True, "scaling": "weak",
@@ -473,30 +481,18 @@ def main():
         "config": {"workload": W16.name, "lattice": "D3Q27", "nx": 512, "ny": 256, "nz": 256,
                    "storage": "fp16 shifted (f_i - w_i rho0)/w_i", "collision": "fp32",
                    "force_interval": 10, "body": "z-cylinder D=40", "Re": 300},
-        "roofline": {"bound": "hbm", "achieved": round(ach16, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": round(ach16 / HBM_PEAK_GBS, 4), "traffic": traffic_from_profiles("fp16s_k_fast_v"),
-                     "kernel": f"k_fast_v<27,SF16,{info16.nodes_per_lane}>", "kernel_ms": round(t16 * 1e3, 5),
-                     "bytes_per_update": info16.bytes_per_update,
-                     "step": {"kernels": "k_fast_v", "ms": round(st16 * 1e3, 5),
-                              "achieved": round(sach16, 1), "frac": round(sach16 / HBM_PEAK_GBS, 4),
-                              "traffic": traffic_from_profiles("fp16s")}},
+        "roofline": kernel_roofline(pkg, L.FP16S, K, info16.bytes_per_update, nodes, "k_pair<SF16>",
+                                    f"k_fast_v<27,SF16,{info16.nodes_per_lane}>", "instruction issue", "fp16s"),
         "forces_finite": bool(forces.size and (abs(forces[:, 1:]) < 1e30).all()),
     }
     if not a.no_fp32:
         log("fp32 leg")
         s32, W32, wall32, info32 = run_leg(pkg, L.FP32, K, Wm, 10)
         s32.close()
-        t32, ach32, st32, sach32 = kernel_roofline(pkg, L.FP32, K, info32.bytes_per_update, nodes)
         out["fp32"] = {"value": round(nodes * K / wall32 / 1e6, 1), "unit": "MLUPS",
                        "ms_per_step": round(wall32 / K * 1e3, 5),
-                       "roofline": {"bound": "hbm", "achieved": round(ach32, 1), "peak": HBM_PEAK_GBS,
-                                    "unit": "GB/s", "frac": round(ach32 / HBM_PEAK_GBS, 4),
-                                    "traffic": traffic_from_profiles("fp32_k_fast_v"),
-                                    "kernel": f"k_fast_v<27,SF32,{info32.nodes_per_lane}>",
-                                    "kernel_ms": round(t32 * 1e3, 5), "bytes_per_update": info32.bytes_per_update,
-                                    "step": {"kernels": "k_fast_v", "ms": round(st32 * 1e3, 5),
-                                             "achieved": round(sach32, 1), "frac": round(sach32 / HBM_PEAK_GBS, 4),
-                                             "traffic": traffic_from_profiles("fp32")}}}
+                       "roofline": kernel_roofline(pkg, L.FP32, K, info32.bytes_per_update, nodes, "k_pair<SF32>",
+                                                   f"k_fast_v<27,SF32,{info32.nodes_per_lane}>", "hbm", "fp32")}
     if not a.no_adjoint:
         log("adjoint leg")
         out["adjoint"] = adjoint_ratio(pkg)

@@ -118,13 +118,13 @@ int lbm_set_ran(lbm_ctx *ctx, const int32_t *ran, size_t count);
 int lbm_initialize(lbm_ctx *ctx);
 
 /* n time steps: the body of main's loop, Collision + pack/exchange/unpack + Streaming +
- * Update (3D MPI+KOKKOS+MPIIO/main.cpp:29-37; lbm.cpp:257-417), one fused kernel per
- * step; asynchronous on the context stream */
+ * Update (3D MPI+KOKKOS+MPIIO/main.cpp:29-37; lbm.cpp:257-417), in fused kernels that advance
+ * one or several steps per launch; asynchronous on the context stream */
 int lbm_step(lbm_ctx *ctx, int n);
 /* the same, bracketed by HIP events on the context stream; *ms = elapsed milliseconds */
 int lbm_step_timed(lbm_ctx *ctx, int n, double *ms);
 /* n steps as lbm_step, timed with HIP events on the context stream: *ms_steps = the n steps,
- * *ms_bulk = the sum over the steps of the bulk kernel alone (k_fast_v; k_dense_v in dense mode;
+ * one per launch, *ms_bulk = the sum over the steps of the bulk kernel alone (k_fast_v; k_dense_v in dense mode;
  * k_fused for FP64 storage), between events recorded just before and after its launch.  Plain mode only,
  * 1 <= n <= 100000.  A measurement entry point with no counterpart in the reference. */
 int lbm_step_kernel_timed(lbm_ctx *ctx, int n, double *ms_steps, double *ms_bulk);
