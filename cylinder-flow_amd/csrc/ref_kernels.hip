@@ -17,7 +17,7 @@
 // every ghost slot into both buffers, so ghost values persist across the swaps exactly as in
 // the reference's single f array -- including the slots no fill ever refreshes.
 #include <algorithm>
-#include <unordered_map>
+#include <vector>
 
 #include "internal.hpp"
 #include "lattice.hpp"
@@ -674,19 +674,28 @@ bool ref_resolve(const RefGeo &r, const std::vector<uint8_t> &usr, std::vector<i
     auto at = [&](int ii, int i, int j) { return ii * plane + i + (long)r.px * j; };   // RIDX in 2D, flat as there
     // the element a copied element's value comes from, after the fills in their order and after usrbc, and
     // the nodes that pull from a node with a copied element (the fills touch the edges, usrbc the body)
-    std::unordered_map<long, int> from;
-    from.reserve(8 * (size_t)(lx + ly));
+    // (nine origins, -1 where none, of each node with a copied element)
+    std::vector<int> block(r.plane, -1), from;
     std::vector<uint8_t> reached(r.plane, 0);
     std::vector<std::pair<long, int>> copies;
+    copies.reserve(6 * (size_t)(lx + ly));
     auto origin = [&](long k) {
-        const auto it = from.find(k);
-        return it == from.end() ? (int)k : it->second;
+        const uint32_t ii = (uint32_t)k / (uint32_t)plane, n = (uint32_t)k - ii * (uint32_t)plane;
+        const int o = block[n] < 0 ? -1 : from[9 * (size_t)block[n] + ii];
+        return o < 0 ? (int)k : o;
     };
     auto copy = [&](long dst, long src) { copies.emplace_back(dst, origin(src)); };
     auto apply = [&]() {   // the copies of one fill read what was there before it
         for (const auto &c : copies) {
-            from[c.first] = c.second;
-            const int n = (int)(c.first % plane), i = n % r.px, j = n / r.px;
+            const uint32_t ii = (uint32_t)c.first / (uint32_t)plane, node = (uint32_t)c.first - ii * (uint32_t)plane;
+            const int i = (int)(node % (uint32_t)r.px), j = (int)(node / (uint32_t)r.px);
+            const bool seen = block[node] >= 0;
+            if (!seen) {
+                block[node] = (int)(from.size() / 9);
+                from.insert(from.end(), 9, -1);
+            }
+            from[9 * (size_t)block[node] + ii] = c.second;
+            if (seen) continue;
             for (int b = std::max(j - 1, 0); b <= std::min(j + 1, ly - 1); b++)
                 for (int a = std::max(i - 1, 0); a <= std::min(i + 1, lx - 1); a++) reached[(size_t)a + (size_t)r.px * b] = 1;
         }
@@ -712,7 +721,8 @@ bool ref_resolve(const RefGeo &r, const std::vector<uint8_t> &usr, std::vector<i
         }
     apply();
     auto interior = [&](int k) {
-        const int n = (int)(k % plane), i = n % r.px, j = n / r.px;
+        const uint32_t n = (uint32_t)k % (uint32_t)plane;
+        const int i = (int)(n % (uint32_t)r.px), j = (int)(n / (uint32_t)r.px);
         return i >= g && i < lx - g && j >= g && j < ly - g;
     };
     special.assign(r.plane, -1);
