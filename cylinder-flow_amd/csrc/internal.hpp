@@ -127,6 +127,9 @@ hipError_t fast_step_f16(int Q, int V, const StepBufs &b, bool force, bool mac, 
 hipError_t fast_step_bf16(int Q, int V, const StepBufs &b, bool force, bool mac, const FusedArgs &a, hipStream_t s);
 // two D3Q27 steps per pass over memory (pair_kernel.hpp): WX x WY columns over runs of cz planes.
 // The words and lists are built once from the mask (pair_plan).
+struct PairSeg {   // the nodes next to the mask among 64 along a row: how many come before them, and which
+    uint32_t base, lo, hi, unused;
+};
 struct PairPlan {
     bool on = false;
     int tiles_x = 0, tiles_y = 0, cz = 0, chunks = 0;
@@ -144,14 +147,20 @@ struct PairPlan {
     int fbx = 0, fgx = 0;
     int nslots = 0;
     double *partials = nullptr;   // force_bytes(nslots)
+    // force of the second step of a pair: the nodes next to the mask (nnear of them) by segment, and with
+    // per-block slots their three sums (else those are the slots)
+    PairSeg *seg = nullptr;
+    int nnear = 0;
+    double *trip = nullptr;
 };
 struct PairOps {   // a storage format's column, LDS bytes and launchers
     int wx, wy;
     size_t lds;
     hipError_t (*prepare)();
     hipError_t (*step)(const PairPlan &p, const void *A, void *B, const void *sfrac, const double *uin, double *macros,
-                       bool mac, const FusedArgs &a, hipStream_t s);
+                       bool mac, double *trip, const FusedArgs &a, hipStream_t s);   // trip: see PairPlan (null: no force)
     hipError_t (*force)(const PairPlan &p, const void *A, double *partials, const FusedArgs &a, hipStream_t s);
+    hipError_t (*block_sum)(const PairPlan &p, double *partials, const FusedArgs &a, hipStream_t s);
 };
 PairOps pair_ops(int prec);
 // the plan of a domain; p.on stays false where the two-step kernel does not apply (pair.cpp).
@@ -160,7 +169,9 @@ PairOps pair_ops(int prec);
 hipError_t pair_plan(PairPlan &p, int prec, const Geo &g, const uint8_t *flags, bool same_offsets, bool packed,
                      const std::vector<uint32_t> &near_nodes, const std::vector<int> &block_slot, Shape blk, hipStream_t s);
 // fills p.bw, p.tflag and p.linklk (pair_words.hip)
-hipError_t pair_words(const PairPlan &p, const PairOps &ops, const uint8_t *flags, const Geo &g, hipStream_t s);
+// masks: per 64 nodes along a row, those next to the mask
+hipError_t pair_words(const PairPlan &p, const PairOps &ops, const uint8_t *flags, unsigned long long *masks, const Geo &g,
+                      hipStream_t s);
 void pair_free(PairPlan &p);
 // several D2Q9 steps per launch (small_kernel.hpp): K steps at most, T x T tiles
 // (tb_choose), tb_tiles(g, T, K) blocks with tb_lds_bytes(prec, T) of LDS each

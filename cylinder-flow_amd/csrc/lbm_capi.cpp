@@ -941,17 +941,25 @@ static int step_n(lbm_ctx *c, int n, hipEvent_t *evs = nullptr) {
         return hipSuccess;
     };
     while (left > 0) {
-        // two steps in one pass unless the second records the force (its input stays in the LDS), or
-        // the first does and a solid fraction carries force (its moments do too); not under
+        // two steps in one pass unless one of them records the force of a solid fraction (its moments
+        // stay in registers), or the second a force that the pass does not sum (pair_plan); not under
         // per-kernel timing
-        if (c->pair.on && !evs && left > 1 && !records(c->step + 2) && !(records(c->step + 1) && c->dsfrac)) {
+        const bool second = records(c->step + 2);
+        if (c->pair.on && !evs && left > 1 && !((second || records(c->step + 1)) && c->dsfrac) && !(second && !c->pair.seg)) {
             const PairOps ops = pair_ops(c->prec);
             if (records(c->step + 1)) {
                 double *partials = nullptr;
                 HIP_TRY(c, next_record(true, c->step + 1, partials));
                 HIP_TRY(c, ops.force(c->pair, c->A, partials, a, c->stream));
             }
-            HIP_TRY(c, ops.step(c->pair, c->A, c->B, c->dsfrac, c->duin, c->macros, false, a, c->stream));
+            double *sums = nullptr, *trip = nullptr;   // of the second step
+            if (second) {
+                HIP_TRY(c, next_record(true, c->step + 2, sums));
+                trip = c->pair.fblk ? c->pair.trip : sums;
+                if (c->pair.nnear == 0) trip = nullptr;
+            }
+            HIP_TRY(c, ops.step(c->pair, c->A, c->B, c->dsfrac, c->duin, c->macros, false, trip, a, c->stream));
+            if (trip && c->pair.fblk) HIP_TRY(c, ops.block_sum(c->pair, sums, a, c->stream));
             c->step += 2;
             left -= 2;
             std::swap(c->A, c->B);
@@ -993,7 +1001,7 @@ int ensure_fields(lbm_ctx *c) {
         else HIP_TRY(c, ref_fused(c->rg, c->rft, c->rf, c->rmac, c->rusr, c->rprof, c->rfpre, c->stream));
     } else {
         const FusedArgs a = ctx_fused_args(c);
-        if (c->replay_pair) HIP_TRY(c, pair_ops(c->prec).step(c->pair, c->B, c->A, c->dsfrac, c->duin, c->macros, true, a, c->stream));
+        if (c->replay_pair) HIP_TRY(c, pair_ops(c->prec).step(c->pair, c->B, c->A, c->dsfrac, c->duin, c->macros, true, nullptr, a, c->stream));
         else HIP_TRY(c, plain_step(c->Q, c->prec, c->V, step_bufs(c, c->B, c->A), false, true, a, c->stream));
     }
     c->fields_fresh = true;

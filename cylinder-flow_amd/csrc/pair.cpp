@@ -18,7 +18,7 @@ PairOps pair_ops(int prec) {
 }
 
 void pair_free(PairPlan &p) {
-    for (void *q : {(void *)p.bw, (void *)p.tflag, (void *)p.link, (void *)p.linklk, (void *)p.link_slot, (void *)p.fblk, (void *)p.partials})
+    for (void *q : {(void *)p.bw, (void *)p.tflag, (void *)p.link, (void *)p.linklk, (void *)p.link_slot, (void *)p.fblk, (void *)p.partials, (void *)p.seg, (void *)p.trip})
         if (q) (void)hipFree(q);
     p = PairPlan{};
 }
@@ -107,7 +107,31 @@ hipError_t pair_plan(PairPlan &p, int prec, const Geo &g, const uint8_t *flags, 
         if (e == hipSuccess) e = upload(p.link_slot, slot);
         if (e == hipSuccess) e = hipMalloc(&p.linklk, sizeof(uint32_t) * (size_t)p.nlink);
     }
-    if (e == hipSuccess) e = pair_words(p, ops, flags, g, s);
+    // the nodes next to the mask by segments of 64
+    std::vector<unsigned long long> masks(g.plane / 64);
+    unsigned long long *dmasks = nullptr;
+    if (e == hipSuccess) e = hipMalloc(&dmasks, sizeof(masks[0]) * masks.size());
+    if (e == hipSuccess) e = pair_words(p, ops, flags, dmasks, g, s);
+    if (e == hipSuccess) e = hipMemcpyAsync(masks.data(), dmasks, sizeof(masks[0]) * masks.size(), hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    if (dmasks) (void)hipFree(dmasks);
+    if (e == hipSuccess) {
+        std::vector<PairSeg> seg(masks.size());
+        size_t n = 0;
+        for (size_t k = 0; k < seg.size(); k++) {
+            seg[k] = {(uint32_t)n, (uint32_t)masks[k], (uint32_t)(masks[k] >> 32), 0u};
+            n += (size_t)__builtin_popcountll(masks[k]);
+        }
+        // The force of a second step is summed in the pass, except in 16 bits next to the packed one-step
+        // kernel, where its instructions cost more than they save: 512x256x256, the force every step, one
+        // launch per step / two steps per pass with it, FP64 2671 / 1753 us per step, FP32 1242 / 864, FP16
+        // 649 / 743.  (The sums are addressed in bytes of 32 bits.)
+        if (n * 24 < ((size_t)1 << 32) && (prec == LBM_FP64 || prec == LBM_FP32 || !packed)) {
+            p.nnear = (int)n;
+            e = upload(p.seg, seg);
+            if (e == hipSuccess && per_block) e = hipMalloc(&p.trip, 24 * std::max<size_t>(n, 1));
+        }
+    }
     if (e == hipSuccess) e = hipMalloc(&p.partials, force_bytes(p.nslots));
     if (e != hipSuccess) {
         pair_free(p);

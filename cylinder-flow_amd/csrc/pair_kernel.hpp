@@ -27,6 +27,11 @@
 // 1.13 times the state), FP16 by instruction issue (68 % VALU busy at 309 instructions per node and
 // step), FP64 by both.
 //
+// A recorded first step's momentum exchange is summed from the pass's input by a kernel of its own
+// (pair_force_s); a second step's by the pass (FORCE): the node's own values are in the LDS when its plane's
+// are pulled, three sums per node next to the mask go to memory by the node's rank (PairSeg).  Those sums
+// and their stores are in every pass's straight line: 3 % of a pass in FP32 and FP64, 29 % in FP16.
+//
 // Every node's arithmetic is that of the one-step kernels (collide, collide_f64, velocity_inlet,
 // the storage format's decode and encode), so populations and fields are theirs bit for bit.
 #pragma once
@@ -159,7 +164,7 @@ __device__ __forceinline__ C pinned(C v) {
 // The march of one block.  A pass k takes plane k from the LDS for the second step and puts plane k + 1 of the first step
 // into it.  The passes are straight-line code in all that touches global memory: a branch around a
 // load or store would make the wait for plane k + 1's loads wait for the stores behind them as well.
-template <class S, bool SFRAC, bool MACROS>
+template <class S, bool SFRAC, bool MACROS, bool FORCE>
 struct PairMarch {
     using L = Lat<27>;
     using T = typename S::T;
@@ -181,6 +186,10 @@ struct PairMarch {
     const C *sfrac;
     const double *uin;
     double *macros;
+    // FORCE: the second step's momentum exchange, three doubles per node next to the mask, in node order
+    const PairSeg *seg;
+    double *trip;
+    uint32_t tripb;   // bytes of trip
     const FusedArgs &a;
     T *lds;
     cword tf;   // bit k of the column's words: plane k holds a bounce word
@@ -197,6 +206,8 @@ struct PairMarch {
     double u1, u2;
     C sf1, sf2;
     uint32_t w1, w2, w2k;
+    uint32_t wally;                    // FORCE: the directions that cross a y wall
+    uint32_t sbase, slo, shi;          // and the segment of the next pass's plane
     T upJ[9], midJ[9], upK[9];   // pulled values of plane k - 1 (e_z > 0, e_z = 0) and of plane k (e_z > 0)
 
     // bounce word of a node of plane k: 0 without a memory access where the plane holds none (the
@@ -204,6 +215,13 @@ struct PairMarch {
     __device__ __forceinline__ uint32_t word(int k, uint32_t node) const {
         const uint32_t on = (tf[k >> 5] >> (k & 31)) & 1u;
         return buf_load<uint32_t>(plane_rsrc(bw + (size_t)planen * k, on * planen * 4u), node * 4u, 0);
+    }
+    template <class F>
+    static constexpr uint32_t dirs(F f) {
+        uint32_t b = 0;
+        for (int i = 1; i < Q; i++)
+            if (f(i)) b |= 1u << i;
+        return b;
     }
     // whether any lane of the wave holds one of these bits
     __device__ __forceinline__ static bool any(uint32_t bits) { return __builtin_amdgcn_ballot_w64(bits != 0u) != 0ull; }
@@ -274,6 +292,12 @@ struct PairMarch {
         node2 = act2 ? (uint32_t)X2 + (uint32_t)g.nxp * (uint32_t)Y2 : 0u;
         out2 = act2 ? (uint32_t)Y2 * rsb + (uint32_t)X2 * esz : ~0u;
         ownv = lds + (DB ? 2 : 1) * Q * NP + (act2 ? cy * WX + cx : 0);   // its node's 9 slots, WX * WY apart
+        if constexpr (FORCE) {
+            wally = 0u;
+            if (!g.yper && Y2 == 0) wally |= dirs([](int i) { return L::ey(i) > 0; });
+            if (!g.yper && Y2 == g.ny - 1) wally |= dirs([](int i) { return L::ey(i) < 0; });
+        }
+        sbase = slo = shi = 0;
         planeb = (uint32_t)(g.rs * (size_t)g.ny * sizeof(T));
         dsb = (uint32_t)(g.ds * sizeof(T));
         static_for<0, Q>([&](auto I) { R[I] = T(0); });
@@ -300,6 +324,15 @@ struct PairMarch {
         if constexpr (SFRAC && FIRST) sf1 = sfrac[node1 + (size_t)planen * kk];
         if constexpr (SFRAC && SECOND) sf2 = sfrac[node2 + (size_t)planen * j];
         if constexpr (SECOND) w2k = word(wrapz(pass + 1), node2);   // of the next pass's plane
+        if constexpr (FORCE && SECOND) {
+            const int n = wrapz(pass + 1);
+            const uint32_t on = (tf[n >> 5] >> (n & 31)) & 1u, segs = planen >> 6;
+            const auto rs = plane_rsrc(seg + (size_t)segs * n, on * segs * (uint32_t)sizeof(PairSeg));
+            const uint32_t at = (node2 >> 6) * (uint32_t)sizeof(PairSeg);
+            sbase = buf_load<uint32_t>(rs, at, 0);
+            slo = buf_load<uint32_t>(rs, at, 4);
+            shi = buf_load<uint32_t>(rs, at, 8);
+        }
         if constexpr (FIRST) {
             const uint32_t w = w1;
             w1 = word(wrapz(k + 1), node1);
@@ -380,6 +413,34 @@ struct PairMarch {
                 else if constexpr (L::ez(i) > 0) upJ[zrank(i)] = pair_pick<T>(w2, i, o, upJ[zrank(i)]);
                 else if (act2) ownv[zrank(i) * WX * WY] = o;
             });
+        if constexpr (FORCE) {
+            // the mask's links of plane k from the node's own values (all of them are in the LDS now), in
+            // direction order; a store that the buffer drops where there are none
+            double f[3] = {0.0, 0.0, 0.0};
+            uint32_t wall = wally;
+            if (!a.g.zper && k == 0) wall |= dirs([](int i) { return L::ez(i) > 0; });
+            if (!a.g.zper && k == a.g.nz - 1) wall |= dirs([](int i) { return L::ez(i) < 0; });
+            const uint32_t links = w2 & ~wall;
+            uint32_t dst = ~0u;
+            if (any(links)) {
+                static_for<1, Q>([&](auto I) {
+                    constexpr int i = I;
+                    constexpr int ex = L::ex(i), ey = L::ey(i), ez = L::ez(i);
+                    const double m = 2.0 * (double)S::template decode<i, L>(in[L::opp(i) * NP + i0], 0.f);
+                    const bool on = (links >> i) & 1u;
+                    if constexpr (ex != 0) f[0] = on ? f[0] - ex * m : f[0];
+                    if constexpr (ey != 0) f[1] = on ? f[1] - ey * m : f[1];
+                    if constexpr (ez != 0) f[2] = on ? f[2] - ez * m : f[2];
+                });
+            }
+            const uint32_t bit = node2 & 63u;
+            const unsigned long long held = (unsigned long long)slo | (unsigned long long)shi << 32;
+            // (a node next to the mask whose links are all clamped away or inlet unknowns stores its zeros)
+            if (act2 && k >= z0 && k < z1 && ((held >> bit) & 1ull))
+                dst = (sbase + (uint32_t)__builtin_popcountll(held & ((1ull << bit) - 1ull))) * 24u;
+            const auto rs = plane_rsrc(trip, tripb);
+            static_for<0, 3>([&](auto D) { buf_store<double>(rs, dst, (uint32_t)D * 8u, f[D]); });
+        }
     }
 
     // passes lo .. hi of a wave with positions of the first step (FIRST), with nodes of the column
@@ -429,11 +490,12 @@ struct PairMarch {
     }
 };
 
-template <class S, bool SFRAC, bool MACROS>
+template <class S, bool SFRAC, bool MACROS, bool FORCE>
 __global__ void __launch_bounds__(PairTile<S>::NT)
     k_pair(const typename S::T *__restrict__ A, typename S::T *__restrict__ B, const uint32_t *__restrict__ bw,
            const uint32_t *__restrict__ tflag, const typename S::C *__restrict__ sfrac, const double *__restrict__ uin,
-           double *__restrict__ macros, const FusedArgs a, int tiles_x, int tiles_y, int cz) {
+           double *__restrict__ macros, const PairSeg *__restrict__ seg, double *__restrict__ trip, uint32_t tripb, const FusedArgs a,
+           int tiles_x, int tiles_y, int cz) {
     extern __shared__ __align__(16) char pair_lds[];
     using T = typename S::T;
     const Geo &g = a.g;
@@ -445,8 +507,8 @@ __global__ void __launch_bounds__(PairTile<S>::NT)
     const int tiles = tiles_x * tiles_y, chunk = __builtin_amdgcn_readfirstlane(pos / tiles), tile = pos - chunk * tiles;
     const int ty = __builtin_amdgcn_readfirstlane(tile / tiles_x);
     const int z0 = chunk * cz, z1 = min(g.nz, z0 + cz);
-    PairMarch<S, SFRAC, MACROS> m{A, B, bw, sfrac, uin, macros, a};
-    typedef typename PairMarch<S, SFRAC, MACROS>::cword cword;
+    PairMarch<S, SFRAC, MACROS, FORCE> m{A, B, bw, sfrac, uin, macros, seg, trip, tripb, a};
+    typedef typename PairMarch<S, SFRAC, MACROS, FORCE>::cword cword;
     m.lds = (T *)pair_lds;
     m.tf = (cword)(uintptr_t)(tflag + (size_t)tile * ((g.nz + 31) / 32));
     m.z0 = z0;
@@ -501,12 +563,41 @@ __global__ void __launch_bounds__(256)
     }
 }
 
+// The same per-block sums from the nodes' own (k_pair, FORCE).
+template <class S>
+__global__ void __launch_bounds__(256)
+    k_block_sum(const PairSeg *__restrict__ seg, const double *__restrict__ trip, const uint32_t *__restrict__ list, int gx,
+                double *__restrict__ partials, Geo g) {
+    const uint32_t id = list[blockIdx.x], row = id / (uint32_t)gx;
+    const uint32_t x = (id - row * (uint32_t)gx) * blockDim.x + threadIdx.x;
+    double fx = 0.0, fy = 0.0, fz = 0.0;
+    if (x < (uint32_t)g.nx) {
+        const PairSeg q = seg[(x + (size_t)g.nxp * row) >> 6];
+        const unsigned long long held = (unsigned long long)q.lo | (unsigned long long)q.hi << 32;
+        const uint32_t bit = x & 63u;
+        if ((held >> bit) & 1ull) {
+            const double *t = trip + 3 * (size_t)(q.base + (uint32_t)__builtin_popcountll(held & ((1ull << bit) - 1ull)));
+            fx = t[0];
+            fy = t[1];
+            fz = t[2];
+        }
+    }
+    __shared__ double red[3 * 4];
+    block_sum3<4>(fx, fy, fz, red);
+    if (threadIdx.x == 0) {
+        partials[3 * (size_t)blockIdx.x] = fx;
+        partials[3 * (size_t)blockIdx.x + 1] = fy;
+        partials[3 * (size_t)blockIdx.x + 2] = fz;
+    }
+}
+
 // ---- launchers of one storage format (pair_f64.hip ... pair_bf16.hip) ----
 template <class S>
 static hipError_t pair_prepare_s() {
     const int bytes = (int)pair_lds_bytes<S>();
-    for (const void *k : {(const void *)k_pair<S, false, false>, (const void *)k_pair<S, false, true>,
-                          (const void *)k_pair<S, true, false>, (const void *)k_pair<S, true, true>}) {
+    for (const void *k : {(const void *)k_pair<S, false, false, false>, (const void *)k_pair<S, false, true, false>,
+                          (const void *)k_pair<S, true, false, false>, (const void *)k_pair<S, true, true, false>,
+                          (const void *)k_pair<S, false, false, true>}) {
         const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
         if (e != hipSuccess) return e;
     }
@@ -515,16 +606,19 @@ static hipError_t pair_prepare_s() {
 
 template <class S>
 static hipError_t pair_step_s(const PairPlan &p, const void *A, void *B, const void *sfrac, const double *uin,
-                              double *macros, bool mac, const FusedArgs &a, hipStream_t s) {
+                              double *macros, bool mac, double *trip, const FusedArgs &a, hipStream_t s) {
     using T = typename S::T;
     using C = typename S::C;
     auto go = [&](auto kern) {
         hipLaunchKernelGGL(kern, dim3((unsigned)(p.tiles_x * p.tiles_y * p.chunks)), dim3(PairTile<S>::NT),
                            (unsigned)pair_lds_bytes<S>(), s, (const T *)A, (T *)B, p.bw, p.tflag, (const C *)sfrac, uin,
-                           macros, a, p.tiles_x, p.tiles_y, p.cz);
+                           macros, p.seg, trip, (uint32_t)(24u * (uint32_t)p.nnear), a, p.tiles_x, p.tiles_y, p.cz);
     };
-    if (sfrac) mac ? go(k_pair<S, true, true>) : go(k_pair<S, true, false>);
-    else mac ? go(k_pair<S, false, true>) : go(k_pair<S, false, false>);
+    if (trip) {
+        if (sfrac || mac) return hipErrorInvalidValue;
+        go(k_pair<S, false, false, true>);
+    } else if (sfrac) mac ? go(k_pair<S, true, true, false>) : go(k_pair<S, true, false, false>);
+    else mac ? go(k_pair<S, false, true, false>) : go(k_pair<S, false, false, false>);
     return hipGetLastError();
 }
 
@@ -542,9 +636,17 @@ static hipError_t pair_force_s(const PairPlan &p, const void *A, double *partial
     return hipGetLastError();
 }
 
+// after a pair whose second step records the force, with per-block slots: p.trip into partials
+template <class S>
+static hipError_t pair_block_sum_s(const PairPlan &p, double *partials, const FusedArgs &a, hipStream_t s) {
+    if (p.nslots == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_block_sum<S>, dim3((unsigned)p.nslots), dim3(p.fbx), 0, s, p.seg, p.trip, p.fblk, p.fgx, partials, a.g);
+    return hipGetLastError();
+}
+
 template <class S>
 constexpr PairOps pair_ops() {
-    return {PairTile<S>::WX, PairTile<S>::WY, pair_lds_bytes<S>(), pair_prepare_s<S>, pair_step_s<S>, pair_force_s<S>};
+    return {PairTile<S>::WX, PairTile<S>::WY, pair_lds_bytes<S>(), pair_prepare_s<S>, pair_step_s<S>, pair_force_s<S>, pair_block_sum_s<S>};
 }
 
 }  // namespace lbm

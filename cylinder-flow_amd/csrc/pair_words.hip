@@ -30,16 +30,19 @@ __device__ __forceinline__ void bounce_word(const uint8_t *__restrict__ flags, c
 // bw of every node; a bit per column and plane whose positions [X0 - 1, X0 + wx] x [Y0 - 1, Y0 + wy]
 // (also through a periodic axis) hold a non-zero word
 __global__ void __launch_bounds__(256) k_pair_words(const uint8_t *__restrict__ flags, uint32_t *__restrict__ bw,
-                                                    uint32_t *__restrict__ tflag, Geo g, int wx, int wy, int tiles_x, int tiles_y) {
+                                                    uint32_t *__restrict__ tflag, unsigned long long *__restrict__ masks, Geo g,
+                                                    int wx, int wy, int tiles_x, int tiles_y) {
     const int x = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y, z = blockIdx.z;
     if (x >= g.nxp) return;
     const size_t node = (size_t)x + (size_t)g.nxp * ((size_t)y + (size_t)g.ny * z);
     uint32_t wall = 0, mask = 0;
     const uint8_t fl = flags[node];   // padding nodes are solid
+    const unsigned long long near = __builtin_amdgcn_ballot_w64(fl == FL_NEAR);   // (rows are multiples of 64 nodes)
+    if ((threadIdx.x & 63u) == 0) masks[node >> 6] = near;
     const bool wallrow = (!g.yper && (y == 0 || y == g.ny - 1)) || (!g.zper && (z == 0 || z == g.nz - 1));
     if (fl != FL_SOLID && (wallrow || fl == FL_NEAR)) bounce_word(flags, g, x, y, z, fl, wall, mask);
     bw[node] = wall | mask;
-    if ((wall | mask) == 0u) return;
+    if ((wall | mask) == 0u && fl != FL_NEAR) return;   // (a node next to the mask has a force slot, links or not)
     const int words = (g.nz + 31) / 32, tx = x / wx, ty = y / wy;
     for (int j = -1; j <= 1; j++)
         for (int i = -1; i <= 1; i++) {
@@ -69,11 +72,12 @@ __global__ void __launch_bounds__(256) k_pair_links(const uint8_t *__restrict__ 
     lk[j] = mask;
 }
 
-hipError_t pair_words(const PairPlan &p, const PairOps &ops, const uint8_t *flags, const Geo &g, hipStream_t s) {
+hipError_t pair_words(const PairPlan &p, const PairOps &ops, const uint8_t *flags, unsigned long long *masks, const Geo &g,
+                      hipStream_t s) {
     hipError_t e = hipMemsetAsync(p.tflag, 0, sizeof(uint32_t) * (size_t)((g.nz + 31) / 32) * p.tiles_x * p.tiles_y, s);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k_pair_words, dim3((unsigned)((g.nxp + 255) / 256), (unsigned)g.ny, (unsigned)g.nz), dim3(256), 0, s, flags,
-                       p.bw, p.tflag, g, ops.wx, ops.wy, p.tiles_x, p.tiles_y);
+                       p.bw, p.tflag, masks, g, ops.wx, ops.wy, p.tiles_x, p.tiles_y);
     if ((e = hipGetLastError()) != hipSuccess || p.nlink == 0) return e;
     hipLaunchKernelGGL(k_pair_links, dim3((unsigned)((p.nlink + 255) / 256)), dim3(256), 0, s, flags, p.link, p.nlink, p.linklk, g);
     return hipGetLastError();
