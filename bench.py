@@ -8,8 +8,8 @@ four side walls, Zou-He inlet (regularised), zero-gradient outlet, drag/lift eve
 initial state (seeded perturbation); the populations are resident in HBM before timing starts.
 
 A "step" is one lattice update of the whole domain.  The solver advances two of them per launch of
-k_pair, which reads and writes the state once; a step whose force is recorded second in its pair, and
-the last of an odd count, run alone in k_fast_v (with k_link_force before it on force steps).
+k_pair, which reads and writes the state once; in FP16 a step whose force is recorded second in its pair,
+and the last of an odd count, run alone in k_fast_v (with k_link_force before it on force steps).
 MLUPS = nodes * steps / seconds over exactly --steps steps bracketed by device synchronisation.  The
 roofline is that of the dominant kernel, k_pair: the algorithmic 2*Q*sizeof(storage) bytes per node
 and launch (two updates) times the nodes, over its launch duration (HIP events around an even number of
