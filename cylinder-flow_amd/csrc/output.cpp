@@ -28,7 +28,8 @@ void output_free(lbm_ctx *c) {
     c->hist_copy.clear();
 }
 
-// a device buffer of at least `elems` doubles and pinned memory for copies of `bytes` bytes
+// a device buffer of at least `elems` doubles and pinned memory for copies of `bytes` bytes (null where
+// there is none to be had: the copies then go straight to the caller's memory)
 static hipError_t reserve(lbm_ctx *c, size_t elems, size_t bytes) {
     if (elems > c->out_elems) {
         if (c->out_dev) (void)hipFree(c->out_dev);
@@ -44,7 +45,11 @@ static hipError_t reserve(lbm_ctx *c, size_t elems, size_t bytes) {
         c->out_pin = nullptr;
         c->out_pinned = 0;
         const hipError_t e = hipHostMalloc((void **)&c->out_pin, pinned, hipHostMallocDefault);
-        if (e != hipSuccess) return e;
+        if (e != hipSuccess) {
+            c->out_pin = nullptr;
+            (void)hipGetLastError();
+            return hipSuccess;
+        }
         c->out_pinned = pinned;
     }
     return hipSuccess;
@@ -52,6 +57,10 @@ static hipError_t reserve(lbm_ctx *c, size_t elems, size_t bytes) {
 
 // `bytes` of device memory into dst, after the stream's work so far; returns when they are there
 static hipError_t copy_out(lbm_ctx *c, void *dst, const void *src, size_t bytes) {
+    if (!c->out_pin) {
+        const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream);
+        return e == hipSuccess ? hipStreamSynchronize(c->stream) : e;
+    }
     if (bytes <= SLICE) {
         hipError_t e = hipMemcpyAsync(c->out_pin, src, bytes, hipMemcpyDeviceToHost, c->stream);
         if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
@@ -112,6 +121,15 @@ hipError_t output_fields(lbm_ctx *c, double *const *outs) {
     if (bytes * n <= SLICE) {   // all of them in one kernel, one copy and one wait
         hipError_t e = reserve(c, c->N * n, bytes * n);
         if (e == hipSuccess) e = gather(want);
+        if (e == hipSuccess && !c->out_pin) {
+            const double *from = c->out_dev;
+            for (int k = 0; k < 4 && e == hipSuccess; k++)
+                if (outs[k]) {
+                    e = copy_out(c, outs[k], from, bytes);
+                    from += c->N;
+                }
+            return e;
+        }
         if (e == hipSuccess) e = hipMemcpyAsync(c->out_pin, c->out_dev, bytes * n, hipMemcpyDeviceToHost, c->stream);
         if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
         if (e != hipSuccess) return e;
