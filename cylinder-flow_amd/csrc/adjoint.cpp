@@ -47,13 +47,14 @@ extern "C" int lbm_adjoint(lbm_ctx *c, int n0, int n1, double scale, int K, doub
     // Freed device memory is cleared before it is given out again, at about 40 GB/s behind the program's
     // back: a program that evaluates gradients one after another runs into that once it has gone through
     // the card's memory, and then pays for every byte of the store (192x96x96 FP32, 400 steps, K = 50, 11.4 GB
-    // per evaluation: 295 ms on average over 80 evaluations, 115 for each of the first 24).  From 4 GB on the
-    // segments are therefore no longer than sqrt(n1) steps, the split with the least states, at the same
-    // recompute; below, what is freed is cleared during the next evaluation, and longer segments leave
-    // fewer remainders of the steps per launch.
-    if ((double)SZ * ((n1 + K - 1) / K + K) >= 4e9) {
-        const int root = (int)std::ceil(std::sqrt((double)n1));
-        if (root < K) K = root;
+    // per evaluation: 295 ms on average over 80 evaluations, 115 for each of the first 24; 209 ms with the split
+    // below; 96x48x48 FP64, 300 steps, 200 evaluations, K = 7 / 20 / 50: 101 / 74 / 110 ms on average, 47 / 70 /
+    // 68 with it).  From 1 GB on the segments are therefore of sqrt(n1) steps where that makes fewer states, at the
+    // same recompute; the copies of the added checkpoints take 1-3 %.  Below, and up to 4 GB where several steps
+    // go into a launch and short segments leave more remainders, the segments are those asked for.
+    {
+        const int root = (int)std::ceil(std::sqrt((double)n1)), states = (n1 + K - 1) / K + K;
+        if ((double)SZ * states >= (c->tb_k >= 2 ? 4e9 : 1e9) && (n1 + root - 1) / root + root < states) K = root;
     }
     const int nseg = (n1 + K - 1) / K;
     int rc = LBM_OK;
@@ -67,6 +68,7 @@ extern "C" int lbm_adjoint(lbm_ctx *c, int n0, int n1, double scale, int K, doub
     std::vector<double> hist;
     size_t freeb = 0, totalb = 0;
 
+    output_free(c);   // the kept output buffer's memory counts as free here
     (void)hipMemGetInfo(&freeb, &totalb);
     // (the store of the segments asked for: what was refused does not depend on the split above)
     const int asked = (n1 + K_asked - 1) / K_asked + K_asked + 2;
